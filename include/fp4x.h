@@ -34,10 +34,11 @@
 extern "C" {
 #endif
 
-#define FP4X_ABI_VERSION 12
+#define FP4X_ABI_VERSION 13
 
 enum {
   FP4X_OK = 0,
+  FP4X_NOT_TAKEN = 1,    /* fp4x_linear_rows: nothing launched, see there */
   FP4X_ERR_ARG = -1,     /* invalid shape, alignment or argument */
   FP4X_ERR_LAUNCH = -2,  /* the HIP runtime rejected a launch */
 };
@@ -106,6 +107,18 @@ int fp4x_w6_linear(const void* x, int64_t x_stride, const void* L, const void* H
  * [nv4_linear -> _nv4, x/fp4x_kernels.py:102-113, :73-99] */
 int fp4x_nv4_linear(const void* x, int64_t x_stride, const void* P, const void* S, float gs, void* out,
                     int out_dtype, int M, int N, int K, int ksplit, float* part, int* tickets, void* stream);
+
+/* The products above for any number of rows M in one launch, by weight format
+ * fmt (FP4X_FMT_MX8, _W8_F32, _W8_F16, _W6, _NV4 or _BF16): w0, w1, s are the
+ * format's planes (w1 only for W6, s none for BF16), gs NVFP4's global scale.
+ * The K sum of an output is split by the kernel, in a fixed order.  Returns
+ * FP4X_NOT_TAKEN, with nothing launched, for what only the entry points of up
+ * to 16 rows take (K not a multiple of 64 but for BF16, a scale plane not
+ * 4-byte aligned, W6's H not 16-byte aligned, K > 2^20, x_stride > 2^23): call
+ * those per 16 rows.
+ * [the same functions, x/fp4x_kernels.py:50-70, :102-113, :147-148, :270-271] */
+int fp4x_linear_rows(int fmt, const void* x, int64_t x_stride, const void* w0, const void* w1, const void* s, float gs,
+                     void* out, int out_dtype, int M, int N, int K, void* stream);
 
 /* y = x . bf16((code - 1.5) * S)^T (times rs[n] when rs != NULL), out [M, N].
  * s_fmt = FP4X_DT_F16 or FP4X_DT_E4M3; G = K / S.shape[1].

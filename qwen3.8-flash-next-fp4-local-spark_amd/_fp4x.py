@@ -12,7 +12,7 @@ import torch  # noqa: F401  (HIP runtime first)
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libfp4x.so")
 
-OK, ERR_ARG, ERR_LAUNCH = 0, -1, -2
+OK, NOT_TAKEN, ERR_ARG, ERR_LAUNCH = 0, 1, -1, -2
 DT_BF16, DT_F32, DT_F16, DT_E4M3 = 0, 1, 2, 3
 FMT_MX8, FMT_W8_F32, FMT_W8_F16, FMT_W6, FMT_NV4, FMT_INT2_F16, FMT_INT2_E4M3, FMT_BF16 = range(8)
 
@@ -29,6 +29,7 @@ _SIGS = {
                               _I),
     "fp4x_w6_linear": ([_P, _I64, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P, _P], _I),
     "fp4x_nv4_linear": ([_P, _I64, _P, _P, _F, _P, _I, _I, _I, _I, _I, _P, _P, _P], _I),
+    "fp4x_linear_rows": ([_I, _P, _I64, _P, _P, _P, _F, _P, _I, _I, _I, _I, _P], _I),
     "fp4x_int2_logits": ([_P, _I64, _P, _P, _I, _P, _P, _I, _I, _I, _I, _I, _P], _I),
     "fp4x_topk_rows": ([_P, _I, _I64, _I, _I, _I, _P, _P, _I64, _P], _I),
     "fp4x_topk_workspace_size": ([_I, _I], _I64),
@@ -54,7 +55,7 @@ _SIGS = {
     "fp4x_read_ceiling": ([_P, _I64, _I, _I, _P, _P], _I),
     "fp4x_hold_cus": ([_I, _I64, _I, _P, _P], _I),
 }
-ABI_VERSION = 12
+ABI_VERSION = 13
 
 _LIB = None
 

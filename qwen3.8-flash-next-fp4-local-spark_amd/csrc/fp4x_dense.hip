@@ -26,6 +26,13 @@ bool launch_w6_stream_one_entry(GemvLaunch p, hipStream_t st);
 bool launch_w6_stream_tile_entry(GemvLaunch p, hipStream_t st);
 bool launch_nv4_stream_tile_entry(GemvLaunch p, hipStream_t st);
 bool launch_mx8_stream_tile_entry(GemvLaunch p, hipStream_t st);
+bool launch_gemm_mx8(const GemvLaunch& p, hipStream_t st);
+bool launch_gemm_w8_f32(const GemvLaunch& p, hipStream_t st);
+bool launch_gemm_w8_f16(const GemvLaunch& p, hipStream_t st);
+bool launch_gemm_w6(const GemvLaunch& p, hipStream_t st);
+bool launch_gemm_nv4(const GemvLaunch& p, hipStream_t st);
+bool launch_gemm_bf16(const GemvLaunch& p, hipStream_t st);
+bool gemm_few_rows(const GemvLaunch& p);
 bool launch_w8_single_stream_f16(GemvLaunch p, hipStream_t st);
 bool launch_w8_single_stream_f32(GemvLaunch p, hipStream_t st);
 int topk_check(const void* logits, int dtype, int64_t stride, int M, int V, int C, void* workspace,
@@ -76,6 +83,7 @@ void reload_switches() {
   w.mx8_stream = on("FP4X_MX8_STREAM");
   w.hc_mix = on("FP4X_HC_MIX");
   w.rows = on("FP4X_ROWS");
+  w.gemm = on("FP4X_GEMM");
   w.hc_xcd = on("FP4X_HC_XCD");
   const char* e = getenv("FP4X_WAVES_PER_CU");
   const int v = e ? atoi(e) : 0;
@@ -208,8 +216,10 @@ int fp4x_mx8_linear(const void* x, int64_t x_stride, const void* w, const void* 
   p.pa.s = static_cast<const uint8_t*>(s);
   if (launch_rows_wide<FmtMX8>(p, (hipStream_t)stream)) return check_launch("mx8_rows");    // 16-20 rows per CU, M = 1
   if (launch_mx8_stream_entry(p, (hipStream_t)stream)) return check_launch("mx8_stream");   // many tiles
+  if (gemm_few_rows(p) && launch_gemm_mx8(p, (hipStream_t)stream)) return check_launch("mx8_gemm");  // M > 8
   if (launch_rows_gemv<FmtMX8>(p, 1, (hipStream_t)stream)) return check_launch("mx8_rows");  // fewer rows
   if (launch_mx8_stream_tile_entry(p, (hipStream_t)stream)) return check_launch("mx8_stream"); // 1/2-1 tile per CU
+  if (ksplit == 1 && launch_gemm_mx8(p, (hipStream_t)stream)) return check_launch("mx8_gemm");
   return launch_gemv_mfma<FmtMX8, EpiStore>(p, 1, (hipStream_t)stream);
 }
 
@@ -221,7 +231,9 @@ int fp4x_bf16_linear(const void* x, int64_t x_stride, const void* w, void* out, 
   if (M == 0 || N == 0) return FP4X_OK;
   GemvLaunch p = base_launch(FP4X_FMT_BF16, x, x_stride, out, out_dtype, N, M, N, K, ksplit, part, tickets);
   p.pa.w0 = static_cast<const uint8_t*>(w);
+  if (gemm_few_rows(p) && launch_gemm_bf16(p, (hipStream_t)stream)) return check_launch("bf16_gemm");  // M > 8
   if (launch_rows_gemv<FmtBF16>(p, 1, (hipStream_t)stream)) return check_launch("bf16_rows");
+  if (ksplit == 1 && launch_gemm_bf16(p, (hipStream_t)stream)) return check_launch("bf16_gemm");
   return launch_gemv_mfma<FmtBF16, EpiStore>(p, 1, (hipStream_t)stream);
 }
 
@@ -249,19 +261,27 @@ int fp4x_w8_linear_layers(const void* x, int64_t x_stride, int64_t x_lstride, co
   // of one workgroup), the mixer's down projection taking the same path; other
   // matrices of few rows (a router gate) or of short rows take the few-rows
   // kernels; other single matrices of at least half a tile per CU stream
-  // through LDS; other shapes use the MFMA core
+  // through LDS; other single matrices without split-K take the blocked GEMM,
+  // and the rest the MFMA core
   hipStream_t st = (hipStream_t)stream;
+  // the mixer's up projection (rows much shorter than they are many) stays on
+  // the core, whose sums the single-launch mixer reproduces bit for bit
+  const bool one = layers == 1 && ksplit == 1 && !(K <= 1024 && N >= 8 * K);
   if (fmt == FP4X_FMT_W8_F16) {
     if (launch_w8_stream<true>(p, layers, st)) return check_launch("w8_stream");
     if (layers == 1 && launch_w8_ktile<true, EpiStore>(p, st)) return check_launch("w8_ktile");
+    if (one && gemm_few_rows(p) && launch_gemm_w8_f16(p, st)) return check_launch("w8_gemm");
     if (launch_rows_gemv<FmtW8<true>>(p, layers, st)) return check_launch("w8_rows");   // few rows (a router gate)
     if (layers == 1 && launch_w8_single_stream_f16(p, st)) return check_launch("w8_single_stream");
+    if (one && launch_gemm_w8_f16(p, st)) return check_launch("w8_gemm");
     return launch_gemv_mfma<FmtW8<true>, EpiStore>(p, layers, st);
   }
   if (launch_w8_stream<false>(p, layers, st)) return check_launch("w8_stream");
   if (layers == 1 && launch_w8_ktile<false, EpiStore>(p, st)) return check_launch("w8_ktile");
+  if (one && gemm_few_rows(p) && launch_gemm_w8_f32(p, st)) return check_launch("w8_gemm");
   if (launch_rows_gemv<FmtW8<false>>(p, layers, st)) return check_launch("w8_rows");
   if (layers == 1 && launch_w8_single_stream_f32(p, st)) return check_launch("w8_single_stream");
+  if (one && launch_gemm_w8_f32(p, st)) return check_launch("w8_gemm");
   return launch_gemv_mfma<FmtW8<false>, EpiStore>(p, layers, st);
 }
 
@@ -283,9 +303,11 @@ int fp4x_w6_linear(const void* x, int64_t x_stride, const void* L, const void* H
   p.pa.s = static_cast<const uint8_t*>(S);
   if (launch_rows_wide<FmtW6>(p, (hipStream_t)stream)) return check_launch("w6_rows");       // many rows, M = 1
   if (launch_w6_stream_entry(p, (hipStream_t)stream)) return check_launch("w6_stream");     // many tiles
+  if (gemm_few_rows(p) && launch_gemm_w6(p, (hipStream_t)stream)) return check_launch("w6_gemm");  // M > 8
   if (launch_rows_gemv<FmtW6>(p, 1, (hipStream_t)stream)) return check_launch("w6_rows");    // fewer rows
   if (launch_w6_stream_one_entry(p, (hipStream_t)stream)) return check_launch("w6_stream");  // 1-2 tiles per CU
   if (launch_w6_stream_tile_entry(p, (hipStream_t)stream)) return check_launch("w6_stream"); // 1/2-1 tile per CU
+  if (ksplit == 1 && launch_gemm_w6(p, (hipStream_t)stream)) return check_launch("w6_gemm");
   return launch_gemv_mfma<FmtW6, EpiStore>(p, 1, (hipStream_t)stream);
 }
 
@@ -300,10 +322,38 @@ int fp4x_nv4_linear(const void* x, int64_t x_stride, const void* P, const void* 
   p.pa.s = static_cast<const uint8_t*>(S);
   p.gs = gs;
   if (launch_nv4_stream_entry(p, (hipStream_t)stream)) return check_launch("nv4_stream");   // many tiles
+  if (gemm_few_rows(p) && launch_gemm_nv4(p, (hipStream_t)stream)) return check_launch("nv4_gemm");  // M > 8
   if (launch_rows_gemv<FmtNV4>(p, 1, (hipStream_t)stream)) return check_launch("nv4_rows");  // fewer rows
   if (launch_nv4_stream_one_entry(p, (hipStream_t)stream)) return check_launch("nv4_stream"); // 1-2 tiles per CU
   if (launch_nv4_stream_tile_entry(p, (hipStream_t)stream)) return check_launch("nv4_stream"); // 1/2-1 tile per CU
+  if (ksplit == 1 && launch_gemm_nv4(p, (hipStream_t)stream)) return check_launch("nv4_gemm");
   return launch_gemv_mfma<FmtNV4, EpiStore>(p, 1, (hipStream_t)stream);
+}
+
+int fp4x_linear_rows(int fmt, const void* x, int64_t x_stride, const void* w0, const void* w1, const void* s, float gs,
+                     void* out, int out_dtype, int M, int N, int K, void* stream) {
+  if (fmt < FP4X_FMT_MX8 || fmt > FP4X_FMT_BF16 || fmt == FP4X_FMT_INT2_F16 || fmt == FP4X_FMT_INT2_E4M3)
+    return fail(FP4X_ERR_ARG, "linear_rows: weight format %lld", fmt);
+  int rc = validate(fmt, x, x_stride, M > 16 ? 16 : M, N, K, 1, nullptr, nullptr);
+  if (rc) return rc;
+  if (!aligned(w0, 16)) return fail(FP4X_ERR_ARG, "linear_rows: weight rows must be 16-byte aligned");
+  if (M == 0 || N == 0) return FP4X_OK;
+  GemvLaunch p = base_launch(fmt, x, x_stride, out, out_dtype, N, M, N, K, 1, nullptr, nullptr);
+  p.pa.w0 = static_cast<const uint8_t*>(w0);
+  p.pa.w1 = fmt == FP4X_FMT_W6 ? static_cast<const uint8_t*>(w1) : nullptr;
+  p.pa.s = static_cast<const uint8_t*>(s);
+  if (fmt == FP4X_FMT_NV4) p.gs = gs;
+  hipStream_t st = (hipStream_t)stream;
+  bool took = false;
+  switch (fmt) {
+    case FP4X_FMT_MX8: took = launch_gemm_mx8(p, st); break;
+    case FP4X_FMT_W8_F32: took = launch_gemm_w8_f32(p, st); break;
+    case FP4X_FMT_W8_F16: took = launch_gemm_w8_f16(p, st); break;
+    case FP4X_FMT_W6: took = launch_gemm_w6(p, st); break;
+    case FP4X_FMT_NV4: took = launch_gemm_nv4(p, st); break;
+    default: took = launch_gemm_bf16(p, st); break;
+  }
+  return took ? check_launch("linear_rows") : FP4X_NOT_TAKEN;
 }
 
 }  // extern "C"

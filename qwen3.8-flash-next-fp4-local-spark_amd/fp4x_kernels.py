@@ -30,7 +30,7 @@ __all__ = [
     "mx8_dequant", "dequant_int2", "dequant_nv4", "dequant_operand", "requantize_mx8", "requantize_nv4", "ORDER",
 ]
 
-MAX_M = 16  # rows per launch; larger M runs as consecutive 16-row launches
+MAX_M = 16  # rows per launch of the decode kernels; the dense linears take more rows in one blocked GEMM launch
 
 
 # ----------------------------------------------------------------- plumbing
@@ -111,14 +111,22 @@ def _check_split(k, cfg, ks_idx=2, bk_idx=1):
     return KS
 
 
-def _linear(fn, fmt, x2, n, k, ks, out_dtype, args):
-    """Run a dense GEMV entry point over 16-row blocks of x2."""
+def _linear(fn, fmt, x2, n, k, ks, out_dtype, args, planes, gs=1.0):
+    """Run a dense linear on x2: up to 16 rows through its GEMV entry point fn,
+    more through the blocked GEMM (planes: w0, w1, s), or in 16-row blocks
+    where that takes no such call."""
     x2 = _act(x2)
     m = x2.shape[0]
     if x2.shape[1] != k:
         raise ValueError(f"fp4x: activation K={x2.shape[1]} does not match weight K={k}")
     out = torch.empty((m, n), dtype=out_dtype, device=x2.device)
     st = _L.stream_of(x2)
+    if m > MAX_M:
+        rc = _L.lib().fp4x_linear_rows(fmt, _ptr(x2), x2.stride(0), *planes, gs, _ptr(out), _dt(out_dtype), m, n, k, st)
+        if rc == _L.OK:
+            return out
+        if rc != _L.NOT_TAKEN:
+            _L.check(rc, "linear_rows")
     for m0 in _rows_blocks(m):
         mb = min(MAX_M, m - m0)
         xb, ob = x2[m0:m0 + mb], out[m0:m0 + mb]
@@ -134,7 +142,8 @@ def mx8_linear(x2, w8, s, cfg, out_dtype=torch.bfloat16):
     _need_cuda(x2, w8, s)
     n, k = w8.shape
     ks = _check_split(k, cfg)
-    return _linear(_L.lib().fp4x_mx8_linear, _L.FMT_MX8, x2, n, k, ks, out_dtype, (_ptr(w8), _ptr(s)))
+    return _linear(_L.lib().fp4x_mx8_linear, _L.FMT_MX8, x2, n, k, ks, out_dtype, (_ptr(w8), _ptr(s)),
+                   (_ptr(w8), None, _ptr(s)))
 
 
 def bf16_linear(x2, w, cfg, out_dtype=torch.bfloat16):
@@ -144,7 +153,8 @@ def bf16_linear(x2, w, cfg, out_dtype=torch.bfloat16):
         w = w.to(torch.bfloat16).contiguous()
     n, k = w.shape
     ks = _check_split(k, cfg)
-    return _linear(_L.lib().fp4x_bf16_linear, _L.FMT_BF16, x2, n, k, ks, out_dtype, (_ptr(w),))
+    return _linear(_L.lib().fp4x_bf16_linear, _L.FMT_BF16, x2, n, k, ks, out_dtype, (_ptr(w),),
+                   (_ptr(w), None, None))
 
 
 def w8_linear(x2, q, s, cfg, out_dtype=torch.bfloat16):
@@ -156,7 +166,8 @@ def w8_linear(x2, q, s, cfg, out_dtype=torch.bfloat16):
     if s.dtype not in (torch.float16, torch.float32):
         raise TypeError("fp4x: W8 scales must be fp32 or fp16")
     fmt = _L.FMT_W8_F16 if sdt == _L.DT_F16 else _L.FMT_W8_F32
-    return _linear(_L.lib().fp4x_w8_linear, fmt, x2, n, k, ks, out_dtype, (_ptr(q), _ptr(s), sdt))
+    return _linear(_L.lib().fp4x_w8_linear, fmt, x2, n, k, ks, out_dtype, (_ptr(q), _ptr(s), sdt),
+                   (_ptr(q), None, _ptr(s)))
 
 
 def w6_linear(x2, L, H, S, cfg, out_dtype=torch.bfloat16):
@@ -164,7 +175,8 @@ def w6_linear(x2, L, H, S, cfg, out_dtype=torch.bfloat16):
     _need_cuda(x2, L, H, S)
     n, k = L.shape[0], L.shape[1] * 2
     ks = _check_split(k, cfg)
-    return _linear(_L.lib().fp4x_w6_linear, _L.FMT_W6, x2, n, k, ks, out_dtype, (_ptr(L), _ptr(H), _ptr(S)))
+    return _linear(_L.lib().fp4x_w6_linear, _L.FMT_W6, x2, n, k, ks, out_dtype, (_ptr(L), _ptr(H), _ptr(S)),
+                   (_ptr(L), _ptr(H), _ptr(S)))
 
 
 def nv4_linear(x2, wp, s, gs, cfg=(32, 256, 4), out_dtype=torch.bfloat16):
@@ -172,7 +184,8 @@ def nv4_linear(x2, wp, s, gs, cfg=(32, 256, 4), out_dtype=torch.bfloat16):
     _need_cuda(x2, wp, s)
     n, k = wp.shape[0], wp.shape[1] * 2
     ks = _check_split(k, cfg, ks_idx=3)
-    return _linear(_L.lib().fp4x_nv4_linear, _L.FMT_NV4, x2, n, k, ks, out_dtype, (_ptr(wp), _ptr(s), float(gs)))
+    return _linear(_L.lib().fp4x_nv4_linear, _L.FMT_NV4, x2, n, k, ks, out_dtype, (_ptr(wp), _ptr(s), float(gs)),
+                   (_ptr(wp), None, _ptr(s)), float(gs))
 
 
 def w8_linear_layers(x3, q3, s3, out_dtype=torch.bfloat16):

@@ -1,0 +1,144 @@
+"""GPU parity of the blocked GEMM (csrc/fp4x_gemm.h): more than 16 rows, and
+the shapes of up to 16 rows that fall to it.
+
+fp32 outputs lie within the MFMA accumulation bound of the exact (float64)
+sum (oracle.ordered.mfma_bound; a K split over up to 10 waves adds as many
+additions as a K split over 10 slices) and bf16 outputs are the same sums
+rounded.  Sizes sit at the edges of its row tiles (16, 32, 48, 64, 128),
+column tiles (16 .. 128), 128-value K units (K = 64 .. 1088, not multiples of
+128) and waves (more waves than units), with odd N.
+"""
+import numpy as np
+import pytest
+import torch
+
+from oracle import formats as fm
+from oracle import gemv as og
+from oracle import ordered
+
+from gpu_helpers import act, bf16_bits, bf16_dev, path_switch, to_f32
+from test_gpu_gemv import prep, run
+
+pytestmark = pytest.mark.gpu
+
+FMTS = ["mx8", "w8", "w8_f16", "w6", "nv4", "bf16"]
+
+
+@pytest.fixture(scope="module")
+def F():
+    import fp4x_kernels
+    return fp4x_kernels
+
+
+def planes_of(fmt, rng, n, k):
+    planes, w_op, gs = prep("w8" if fmt == "w8_f16" else fmt, rng, n, k)
+    if fmt == "w8_f16":
+        planes = (planes[0], planes[1].half())
+        w_op = og.operand("w8", planes[0].cpu().numpy(), planes[1].float().cpu().numpy())
+    return planes, w_op, gs
+
+
+def check(F, fmt, planes, w_op, gs, x, xd):
+    base = "w8" if fmt == "w8_f16" else fmt
+    y = to_f32(run(F, base, xd, planes, 1, torch.float32))
+    exact = ordered.exact_sum(x, w_op) * gs
+    bound = ordered.mfma_bound(x, w_op, 10) * abs(gs)
+    assert np.all(np.abs(y - exact) <= bound), (np.abs(y - exact) / bound).max()
+    assert np.array_equal(bf16_bits(run(F, base, xd, planes, 1)), fm.bf16_bits(y))
+    return y
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("M,N,K", [(17, 1, 64), (17, 33, 192), (24, 640, 640), (31, 1000, 1088), (40, 130, 2560),
+                                   (48, 4100, 576), (65, 97, 1344), (100, 513, 320), (129, 301, 128), (200, 8200, 256),
+                                   (256, 1025, 704)])
+def test_gemm_rows(gpu, F, fmt, M, N, K):
+    rng = np.random.default_rng(M + N + K)
+    planes, w_op, gs = planes_of(fmt, rng, N, K)
+    x, _ = act(rng, M, K)
+    y = check(F, fmt, planes, w_op, gs, x, bf16_dev(x))
+    # rows of x further apart than K, in the middle of another tensor
+    wide = torch.full((M + 2, K + 24), float("nan"), dtype=torch.bfloat16, device="cuda")
+    wide[1:-1, 8:K + 8] = bf16_dev(x)
+    y2 = to_f32(run(F, "w8" if fmt == "w8_f16" else fmt, wide[1:-1, 8:K + 8], planes, 1, torch.float32))
+    assert np.array_equal(y.view(np.uint32), y2.view(np.uint32))
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("M,N,K", [(3, 7001, 1920), (5, 1280, 2560), (9, 512, 2560), (13, 96, 1088), (16, 2560, 6144),
+                                   (16, 2560, 640), (16, 5000, 1984)])
+def test_gemm_up_to_16_rows(gpu, F, fmt, M, N, K, monkeypatch):
+    """The shapes of up to 16 rows that fall to it, against the exact sums;
+    FP4X_GEMM=0 (the MFMA core or the few-rows kernel) stays within the same
+    bound."""
+    rng = np.random.default_rng(M + N + K)
+    planes, w_op, gs = planes_of(fmt, rng, N, K)
+    x, _ = act(rng, M, K)
+    check(F, fmt, planes, w_op, gs, x, bf16_dev(x))
+    with path_switch(monkeypatch, "FP4X_GEMM"):
+        check(F, fmt, planes, w_op, gs, x, bf16_dev(x))
+
+
+def test_gemm_bf16_short_tail(gpu, F):
+    """K a multiple of 16 only (bf16)."""
+    rng = np.random.default_rng(5)
+    planes, w_op, gs = planes_of("bf16", rng, 75, 208)
+    x, _ = act(rng, 37, 208)
+    xd = bf16_dev(x)
+    y = to_f32(F.bf16_linear(xd, *planes, (32, 16, 1, 4), torch.float32))
+    assert np.all(np.abs(y - ordered.exact_sum(x, w_op)) <= ordered.mfma_bound(x, w_op, 10))
+
+
+@pytest.mark.parametrize("M", [3, 20, 70])
+def test_gemm_special_values(gpu, F, M):
+    """MXFP8 exponent 255 (scale +inf) gives +-inf or NaN in its own columns
+    only, NaN and inf activations reach their own rows only, as one launch per
+    16 rows gives them; K not a multiple of 128, N odd."""
+    rng = np.random.default_rng(M)
+    N, K = 3001, 1088                                # few rows of 64 tiles, many units
+    (w, s), _, _ = prep("mx8", rng, N, K)
+    s = s.clone()
+    s[7, 3] = 255
+    s[N - 1, K // 32 - 1] = 255
+    x = torch.from_numpy(rng.standard_normal((M, K)).astype(np.float32)).to("cuda").to(torch.bfloat16)
+    x[1, 40] = float("inf")
+    x[2, K - 1] = float("nan")
+    got = F.mx8_linear(x, w, s, (32, 64, 1, 4), torch.float32)
+    want = torch.cat([x[m:m + 1].double() @ F.dequant_operand("mx8", w, None, s, K=K).double().T for m in range(M)])
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(torch.isinf(got), torch.isinf(want))
+    inf = torch.isinf(want)
+    assert torch.equal(got[inf].double(), want[inf])
+    assert not torch.isfinite(got[:, 7]).any() and torch.isfinite(got[0, 8:N - 1]).all()
+
+
+def test_gemm_unaligned_falls_back(gpu, F):
+    """Scales that are only 2-byte aligned take the 16-row launches, with the
+    same results as an aligned copy within the bound."""
+    rng = np.random.default_rng(9)
+    (P, S, gs), w_op, _ = prep("nv4", rng, 260, 640)
+    buf = torch.zeros(S.numel() + 2, dtype=torch.uint8, device="cuda")
+    buf[2:] = S.view(torch.uint8).view(-1)
+    S2 = buf[2:].view(S.shape).view(torch.float8_e4m3fn)
+    assert S2.data_ptr() % 4 == 2
+    x, _ = act(rng, 21, 640)
+    for scales in (S, S2):
+        y = to_f32(F.nv4_linear(bf16_dev(x), P, scales, gs, (32, 64, 4), torch.float32))
+        assert np.all(np.abs(y - ordered.exact_sum(x, w_op) * gs) <= ordered.mfma_bound(x, w_op, 10) * gs)
+
+
+def test_gemm_graph(gpu, F):
+    """Captured and replayed with the program's own work in between."""
+    rng = np.random.default_rng(11)
+    planes, _, _ = planes_of("w6", rng, 1000, 1088)
+    x = bf16_dev(act(rng, 50, 1088)[0])
+    want = run(F, "w6", x, planes, 1)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        y = run(F, "w6", x, planes, 1)
+    for _ in range(3):
+        y.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)
+        assert torch.equal(run(F, "w6", x, planes, 1), want)
