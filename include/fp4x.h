@@ -245,6 +245,12 @@ int fp4x_quantize_w6_clip(int src, const void* src_a, const void* src_b, float s
  * float the caller zeroes first.  [quantize_nv4's global amax, x/fp4x_kernels.py:284-287] */
 int fp4x_absmax(int src, const void* src_a, const void* src_b, float src_gs, int64_t N, int K, float* out,
                 void* stream);
+/* fp4x_absmax into *amax (a device float the caller zeroes first), then the
+ * NVFP4 target with the global scale max(*amax / 6 / 448, 1e-30) worked out on
+ * the device, so the caller need not wait for *amax in between.
+ * [quantize_nv4, x/fp4x_kernels.py:277-300] */
+int fp4x_quantize_nv4(int src, const void* src_a, const void* src_b, float src_gs, int64_t N, int K, float* amax,
+                      void* P, void* S, void* stream);
 
 /* Mixer down projection: split-K W8 GEMV whose last workgroup per row tile
  * writes di = bf16(sum) [M, N] and bot = bf16(sc * sigmoid(sc)) [M, lr] with

@@ -1,7 +1,9 @@
 // Weight preparation on the device: the reference's pure-torch quantizers
 // (x/fp4x_kernels.py: quantize_w8 :138-144, quantize_w6 :179-202 with or
 // without the clip search, quantize_nv4 :277-300, quantize_int2 :330-351 with fp16 scales,
-// or e4m3 scales under an fp32 row scale) as one thread per quantization group.
+// or e4m3 scales under an fp32 row scale) as one thread per 16 weights: the
+// 1, 2 or 4 lanes of a quantization group share its maximum.  (One thread per
+// group for the clip search, one wave per row for the e4m3 INT2 target.)
 //
 // The source rows are fp32, bf16, or packed MXFP8 / NVFP4 rows decoded in
 // registers with the exact dequant of mx8_dequant (:261-267) or dequant_nv4
@@ -10,7 +12,15 @@
 // Arithmetic follows the reference's formulas with IEEE fp32 division, the
 // semantics of its torch ops on CPU tensors (where its golden vectors were
 // taken): torch's GPU division by a Python scalar multiplies by the
-// reciprocal instead, which can move a result by one fp32 ulp.
+// reciprocal instead, which can move a result by one fp32 ulp.  A division per
+// weight is about 11 instructions, and was what these kernels spent their time
+// on; exact_quot gives the same quotient in 3 from the scale's reciprocal, and
+// the INT2 codes need comparisons only.  Groups with infinities, NaN or scales
+// at the ends of their range still divide.  us, before -> after, kernels alone
+// (MXFP8 rows): the 248,320 x 2560 head's INT2 copy 396 -> 186 (893 MB);
+// [16384 x 2560] to W8 33 -> 15, to W6 34 -> 18, to NVFP4 44 -> 20, its
+// global maximum 99 -> 11 (one atomic per workgroup that raises it, instead
+// of one per wave, all on one word).
 #include <cmath>
 
 #include "fp4x_kernels.h"
@@ -22,9 +32,12 @@ int device_cus();
 
 // ------------------------------------------------------------------ sources
 // load<G>(row, k0, f): the G fp32 weights [k0, k0 + G) of a row (k0 % 16 == 0).
+// load16(t, f): weights [16 t, 16 t + 16) of the whole matrix (every plane is
+// one run of memory, K being a multiple of 64).
 struct SrcF32 {
   const float* w;
   int64_t ld;
+  __device__ void load16(int64_t t, float (&f)[16]) const { SrcF32{w + 16 * t, 0}.load<16>(0, 0, f); }
   template <int G>
   __device__ void load(int64_t row, int k0, float (&f)[G]) const {
     const float4* p = reinterpret_cast<const float4*>(w + row * ld + k0);
@@ -39,6 +52,7 @@ struct SrcF32 {
 struct SrcBF16 {
   const uint16_t* w;
   int64_t ld;
+  __device__ void load16(int64_t t, float (&f)[16]) const { SrcBF16{w + 16 * t, 0}.load<16>(0, 0, f); }
   template <int G>
   __device__ void load(int64_t row, int k0, float (&f)[G]) const {
     const uint4* p = reinterpret_cast<const uint4*>(w + row * ld + k0);
@@ -60,6 +74,7 @@ struct SrcMX8 {
   const uint8_t* w;
   const uint8_t* s;
   int K;
+  __device__ void load16(int64_t t, float (&f)[16]) const { SrcMX8{w + 16 * t, s + (t >> 1), 32}.load<16>(0, 0, f); }
   template <int G>
   __device__ void load(int64_t row, int k0, float (&f)[G]) const {
 #pragma unroll
@@ -91,6 +106,7 @@ struct SrcNV4 {
   const uint8_t* S;
   float gs;
   int K;
+  __device__ void load16(int64_t t, float (&f)[16]) const { SrcNV4{P + 8 * t, S + t, gs, 16}.load<16>(0, 0, f); }
   template <int G>
   __device__ void load(int64_t row, int k0, float (&f)[G]) const {
 #pragma unroll
@@ -137,40 +153,122 @@ __device__ __forceinline__ float group_amax(const float (&f)[G]) {
   return a;
 }
 
+// Maximum of |f| over the 16 LPG weights of a group's LPG lanes (1, 2 or 4
+// neighbours); a NaN weight makes it NaN (v_maximum3_f32).
+template <int CTRL>
+__device__ __forceinline__ float dpp_f32(float v) {
+  return __uint_as_float((uint32_t)__builtin_amdgcn_mov_dpp((int)__float_as_uint(v), CTRL, 0xf, 0xf, true));
+}
+template <int LPG>
+__device__ __forceinline__ float lanes_maximum(const float (&f)[16]) {
+  float a = fabsf(f[0]);
+#pragma unroll
+  for (int i = 1; i < 16; ++i) a = __builtin_elementwise_maximum(a, fabsf(f[i]));
+  if constexpr (LPG >= 2) a = __builtin_elementwise_maximum(a, dpp_f32<0xB1>(a));   // lane ^ 1
+  if constexpr (LPG >= 4) a = __builtin_elementwise_maximum(a, dpp_f32<0x4E>(a));   // lane ^ 2
+  return a;
+}
+// The reference's maximum, which skips NaN weights.
+template <int LPG>
+__device__ __forceinline__ float lanes_amax(const float (&f)[16]) {
+  float a = group_amax(f);
+  if constexpr (LPG >= 2) a = fmaxf(a, dpp_f32<0xB1>(a));
+  if constexpr (LPG >= 4) a = fmaxf(a, dpp_f32<0x4E>(a));
+  return a;
+}
+__device__ __forceinline__ bool finite_max(float m) { return m < __builtin_inff(); }   // false for NaN
+
+// Targets: put(t, f) quantizes weights [16 t, 16 t + 16) of the matrix; lanes
+// t of one group run together.
+constexpr float kRint = 12582912.0f;               // 1.5 * 2^23: v + kRint holds rint(v) in its low bits
+
+// RN(f / s) from rs = RN(1 / s) (Markstein: a quotient within an ulp, its exact
+// remainder by fma, and one correction with the rounded reciprocal give the
+// rounded quotient), for 2^-100 <= s < 2^100 and finite f; a quotient so small
+// that the remainder underflows is still within an ulp, which no code notices.
+// -0 gives +0.
+__device__ __forceinline__ float exact_quot(float f, float s, float rs) {
+  const float q = f * rs;
+  return __builtin_fmaf(__builtin_fmaf(-q, s, f), rs, q);
+}
+__device__ __forceinline__ bool mid_range(float s) { return s >= 0x1p-100f && s < 0x1p100f; }
+
 // ------------------------------------------------------------------ targets
 // W8 g64: s = max(amax, 1e-12) / 127, q = clamp(rint(w / s), -127, 127).
+// The clamp never acts on a finite group: its maximum gives 127.
 struct QW8 {
-  static constexpr int G = 64;
+  static constexpr int G = 64, LPG = 4;
   int8_t* q;
   float* s;
-  __device__ void put(int64_t row, int gi, int K, const float (&f)[G]) const {
-    const float sc = fmaxf(group_amax(f), 1e-12f) / 127.0f;
-    uint32_t w[16];
+  __device__ void put(int64_t t, const float (&f)[16]) const {
+    float m = lanes_maximum<LPG>(f);
+    const bool fin = finite_max(m);
+    if (!fin) m = lanes_amax<LPG>(f);
+    const float sc = fmaxf(m, 1e-12f) / 127.0f;
+    uint32_t b[16];
+    if (fin && mid_range(sc)) {
+      const float rc = 1.0f / sc;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      uint32_t b = 0;
+      for (int i = 0; i < 16; ++i) b[i] = __float_as_uint(exact_quot(f[i], sc, rc) + kRint);
+    } else {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float r = fminf(fmaxf(rintf(f[4 * i + j] / sc), -127.0f), 127.0f);
-        b |= ((uint32_t)(int)r & 0xffu) << (8 * j);
-      }
-      w[i] = b;
+      for (int i = 0; i < 16; ++i) b[i] = (uint32_t)(int)fminf(fmaxf(rintf(f[i] / sc), -127.0f), 127.0f);
     }
-    uint4* o = reinterpret_cast<uint4*>(q + row * K + gi * G);
+    uint32_t w[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) o[i] = make_uint4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]);
-    s[row * (K / G) + gi] = sc;
+    for (int i = 0; i < 4; ++i)
+      w[i] = perm_b32(perm_b32(b[4 * i + 3], b[4 * i + 2], 0x0c0c0400u), perm_b32(b[4 * i + 1], b[4 * i], 0x0c0c0400u),
+                      0x05040100u);
+    reinterpret_cast<uint4*>(q)[t] = make_uint4(w[0], w[1], w[2], w[3]);
+    if ((t & 3) == 0) s[t >> 2] = sc;
   }
 };
 
 // W6 g32: s = max(fp16(amax / qmax), 6.2e-5), c = clamp(rint(w / s), -qmax-1,
 // qmax) + 32, split into the nibble plane L and the bit-pair plane H.
-struct QW6 {
-  static constexpr int G = 32;
+struct W6Planes {
   uint8_t* L;
   uint8_t* H;
   uint16_t* S;
   int qmax;
+};
+// By 16 weights.  fp16's rounding of the scale moves the quotient of a finite
+// group's maximum by at most 2^-11 of it (a scale raised to 6.2e-5 makes
+// quotients smaller), so the clamp never acts.
+struct QW6 : W6Planes {
+  static constexpr int G = 32, LPG = 2;
+  __device__ void put(int64_t t, const float (&f)[16]) const {
+    float m = lanes_maximum<LPG>(f);
+    const bool fin = finite_max(m);
+    if (!fin) m = lanes_amax<LPG>(f);
+    const float sc = fmaxf(f16_round(m / (float)qmax), 6.2e-5f);
+    uint32_t c[16];
+    if (fin && finite_max(sc)) {                   // (fp16 can overflow)
+      const float rc = 1.0f / sc;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) c[i] = __float_as_uint(exact_quot(f[i], sc, rc) + (kRint + 32.0f));
+    } else {
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        c[i] = (uint32_t)((int)fminf(fmaxf(rintf(f[i] / sc), (float)(-qmax - 1)), (float)qmax) + 32);
+    }
+    uint32_t l[2] = {0, 0}, h = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {                  // four codes a byte each, then their nibbles and bit pairs
+      const uint32_t b = perm_b32(perm_b32(c[4 * i + 3], c[4 * i + 2], 0x0c0c0400u),
+                                  perm_b32(c[4 * i + 1], c[4 * i], 0x0c0c0400u), 0x05040100u);
+      const uint32_t n = b & 0x0f0f0f0fu, n2 = n | (n >> 4), p = (b >> 4) & 0x03030303u;
+      l[i >> 1] |= ((n2 & 0xffu) | ((n2 >> 8) & 0xff00u)) << (16 * (i & 1));
+      h |= ((p | (p >> 14) | (p >> 4) | (p >> 18)) & 0xffu) << (8 * i);
+    }
+    reinterpret_cast<uint2*>(L)[t] = make_uint2(l[0], l[1]);
+    reinterpret_cast<uint32_t*>(H)[t] = h;
+    if ((t & 1) == 0) S[t >> 1] = __builtin_bit_cast(uint16_t, (_Float16)sc);
+  }
+};
+// By groups.
+struct QW6Group : W6Planes {
+  static constexpr int G = 32;
   __device__ static float base_scale(const float (&f)[G], int qmax) {
     return fmaxf(f16_round(group_amax(f) / (float)qmax), 6.2e-5f);
   }
@@ -192,9 +290,6 @@ struct QW6 {
     *reinterpret_cast<uint4*>(L + row * (K / 2) + gi * 16) = make_uint4(l[0], l[1], l[2], l[3]);
     *reinterpret_cast<uint2*>(H + row * (K / 4) + gi * 8) = make_uint2(h[0], h[1]);
     S[row * (K / G) + gi] = __builtin_bit_cast(uint16_t, (_Float16)sc);
-  }
-  __device__ void put(int64_t row, int gi, int K, const float (&f)[G]) const {
-    put_scaled(row, gi, K, f, base_scale(f, qmax));
   }
 };
 
@@ -225,7 +320,7 @@ __device__ __forceinline__ float w6_sq_err(const float (&f)[32], float sc, int q
   for (int j = 1; j < 8; ++j) e = e + lane[j];
   return e;
 }
-struct QW6Clip : QW6 {
+struct QW6Clip : QW6Group {
   W6Clip clip;
   __device__ void put(int64_t row, int gi, int K, const float (&f)[G]) const {
 #pragma clang fp contract(off)
@@ -250,26 +345,55 @@ struct QW6Clip : QW6 {
 
 // NVFP4 g16: sc = e4m3(clamp(amax / 6 / gs, 2^-9, 448)), v = clamp(w / (sc * gs),
 // -6, 6), magnitude = the number of e2m1 midpoints below |v| (ties go down),
-// sign bit 3 for v < 0.
+// sign bit 3 for v < 0.  The e2m1 conversion rounds ties to even, which goes up
+// at 0.75, 1.75 and 3.5 alone of the midpoints, those whose leading fraction bit
+// is set: one fp32 step less for such quotients sends them down and moves no
+// other quotient across a midpoint.  Taken for sf in [2^-100, 1), where no
+// nonzero quotient underflows to a zero (whose sign would be lost), and amax <=
+// 6.9 sf, where the conversion rounds to 6 by itself.
+__device__ __forceinline__ float nv4_global_scale(float amax) {
+  return (float)fmax((double)amax / 6.0 / 448.0, 1e-30);   // as the host computes it
+}
 struct QNV4 {
-  static constexpr int G = 16;
+  static constexpr int G = 16, LPG = 1;
   uint8_t* P;
   uint8_t* S;
   float gs;
-  __device__ void put(int64_t row, int gi, int K, const float (&f)[G]) const {
-    const float sc = fminf(fmaxf(group_amax(f) / 6.0f / gs, 0x1p-9f), 448.0f);
+  __device__ void put(int64_t t, const float (&f)[16]) const { put_gs(t, f, gs); }
+  __device__ void put_gs(int64_t t, const float (&f)[16], float gsv) const {
+    float m = lanes_maximum<1>(f);
+    const bool fin = finite_max(m);
+    if (!fin) m = group_amax(f);
+    const float sc = fminf(fmaxf(m / 6.0f / gsv, 0x1p-9f), 448.0f);
     const uint32_t code = e4m3_code(sc);
-    const float sf = e4m3_value(code) * gs;
+    const float sf = e4m3_value(code) * gsv;
     uint32_t p[2] = {0, 0};
+    if (fin && sf >= 0x1p-100f && sf < 1.0f && m <= 6.9f * sf) {
+      const float rs = 1.0f / sf;
+      float v[16];
 #pragma unroll
-    for (int i = 0; i < G; ++i) {
-      const float v = fminf(fmaxf(f[i] / sf, -6.0f), 6.0f), a = fabsf(v);
-      const uint32_t mag = (a > 0.25f) + (a > 0.75f) + (a > 1.25f) + (a > 1.75f) + (a > 2.5f) + (a > 3.5f) +
-                           (a > 5.0f);
-      p[i >> 3] |= (mag | (v < 0.0f ? 8u : 0u)) << (4 * (i & 7));
+      for (int i = 0; i < 16; ++i) {
+        const uint32_t b = __float_as_uint(exact_quot(f[i], sf, rs));
+        v[i] = __uint_as_float(b - ((b >> 22) & 1u));
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        p[h] = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(p[h], v[8 * h], v[8 * h + 1], 1.0f, 0);
+        p[h] = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(p[h], v[8 * h + 2], v[8 * h + 3], 1.0f, 1);
+        p[h] = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(p[h], v[8 * h + 4], v[8 * h + 5], 1.0f, 2);
+        p[h] = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(p[h], v[8 * h + 6], v[8 * h + 7], 1.0f, 3);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < G; ++i) {
+        const float v = fminf(fmaxf(f[i] / sf, -6.0f), 6.0f), a = fabsf(v);
+        const uint32_t mag = (a > 0.25f) + (a > 0.75f) + (a > 1.25f) + (a > 1.75f) + (a > 2.5f) + (a > 3.5f) +
+                             (a > 5.0f);
+        p[i >> 3] |= (mag | (v < 0.0f ? 8u : 0u)) << (4 * (i & 7));
+      }
     }
-    *reinterpret_cast<uint2*>(P + row * (K / 2) + gi * 8) = make_uint2(p[0], p[1]);
-    S[row * (K / G) + gi] = (uint8_t)code;
+    reinterpret_cast<uint2*>(P)[t] = make_uint2(p[0], p[1]);
+    S[t] = (uint8_t)code;
   }
 };
 
@@ -292,17 +416,42 @@ __device__ __forceinline__ void put_int2_codes(const float (&f)[G], float sf, ui
   for (int i = 0; i < G / 16; ++i) o32[i] = b[i];
 }
 
+// The 16 codes of one word without a division, for finite weights and a normal
+// scale 0 < sf < 2: the rounded quotient reaches 1 exactly where w >= sf and
+// stays above -1 exactly where w >= -sf (the quotients of sf's two fp32
+// neighbours round to 1 - 2^-24 or less and to 1 + 2^-23), and it keeps the
+// sign of w (nothing underflows to zero).  So 3 - code has the bits (w < 0, w -
+// copysign(sf, w) < 0), shifted in from the last element's to the first's.
+__device__ __forceinline__ uint32_t int2_word(const float (&f)[16], float sf) {
+  uint32_t acc = 0;
+#pragma unroll
+  for (int b = 3; b >= 0; --b)
+#pragma unroll
+    for (int j = 3; j >= 0; --j) {                 // bit pairs 3..0 hold elements 3, 1, 2, 0
+      const int i = 4 * b + (j == 1 ? 2 : j == 2 ? 1 : j);
+      const float w = f[i] + 0.0f;                 // -0 as +0
+      acc = __builtin_amdgcn_alignbit(acc, __float_as_uint(w), 31);
+      acc = __builtin_amdgcn_alignbit(acc, __float_as_uint(w - __builtin_copysignf(sf, w)), 31);
+    }
+  return ~acc;
+}
+
 // INT2 with fp16 group scales: s = fp16(max(amax, 1e-8) / 1.5) (a zero group's
 // scale underflows fp16 to 0, and its codes are 0).
 template <int GG>
 struct QInt2 {
-  static constexpr int G = GG;
+  static constexpr int G = GG, LPG = GG / 16;
   uint8_t* P;
   uint16_t* S;
-  __device__ void put(int64_t row, int gi, int K, const float (&f)[G]) const {
-    const _Float16 s16 = (_Float16)(fmaxf(group_amax(f), 1e-8f) / 1.5f);
-    put_int2_codes(f, (float)s16, P + row * (K / 4) + gi * (G / 4));
-    S[row * (K / G) + gi] = __builtin_bit_cast(uint16_t, s16);
+  __device__ void put(int64_t t, const float (&f)[16]) const {
+    float m = lanes_maximum<LPG>(f);
+    const bool fin = finite_max(m);
+    if (!fin) m = lanes_amax<LPG>(f);
+    const _Float16 s16 = (_Float16)(fmaxf(m, 1e-8f) / 1.5f);
+    const float sf = (float)s16;
+    if (fin && sf > 0.0f && sf < 2.0f) reinterpret_cast<uint32_t*>(P)[t] = int2_word(f, sf);
+    else put_int2_codes<16>(f, sf, P + 4 * t);
+    if (t % LPG == 0) S[t / LPG] = __builtin_bit_cast(uint16_t, s16);
   }
 };
 
@@ -325,8 +474,9 @@ struct QInt2E {
   }
 };
 
+// One thread per group (the clip search).
 template <class Src, class Q>
-__global__ __launch_bounds__(256) void quant_kernel(Src src, Q q, int64_t N, int K) {
+__global__ __launch_bounds__(256) void quant_group_kernel(Src src, Q q, int64_t N, int K) {
   const int gpr = K / Q::G;
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= N * gpr) return;
@@ -337,22 +487,68 @@ __global__ __launch_bounds__(256) void quant_kernel(Src src, Q q, int64_t N, int
   q.put(row, gi, K, f);
 }
 
-// max |w| over the whole matrix into *out (zeroed by the caller): per-thread
-// maxima over 16-groups, a wave maximum, one atomic max of the fp32 bits
-// (ordered as unsigned for non-negative values) per wave.
+// One thread per 16 weights; n16 (a multiple of 4, so of every LPG) of them.
+template <class Src, class Q>
+__global__ __launch_bounds__(256) void quant_kernel(Src src, Q q, int64_t n16) {
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (t >= n16) return;
+  float f[16];
+  src.load16(t, f);
+  q.put(t, f);
+}
+
+// The NVFP4 target with the global scale of *amax, worked out once per workgroup.
 template <class Src>
-__global__ __launch_bounds__(256) void absmax_kernel(Src src, int64_t N, int K, uint32_t* out) {
-  const int64_t groups = N * (K / 16);
-  float m = 0.0f;
-  for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < groups; t += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t row = t / (K / 16);
+__global__ __launch_bounds__(256) void quant_nv4_amax_kernel(Src src, QNV4 q, int64_t n16, const float* amax) {
+  __shared__ float gs;
+  if (threadIdx.x == 0) gs = nv4_global_scale(*amax);
+  __syncthreads();
+  for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < n16; t += (int64_t)gridDim.x * 256) {
     float f[16];
-    src.template load<16>(row, (int)(t - row * (K / 16)) * 16, f);
+    src.load16(t, f);
+    q.put_gs(t, f, gs);
+  }
+}
+
+// max |w| over the whole matrix into *out (zeroed by the caller): per-thread
+// maxima over pieces of 16 weights, the workgroup's maximum, and an atomic max
+// of its fp32 bits (ordered as unsigned for non-negative values) where it is
+// above what *out already holds: atomics on one word queue, about 10 ns each.
+template <class Src>
+__global__ __launch_bounds__(512) void absmax_kernel(Src src, int64_t n16, uint32_t* out) {
+  __shared__ float part[8];
+  const int64_t step = (int64_t)gridDim.x * 512;
+  float m = 0.0f;
+  int64_t t = (int64_t)blockIdx.x * 512 + threadIdx.x;
+  for (; t + 3 * step < n16; t += 4 * step) {          // four pieces in flight
+    float f[4][16];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) src.load16(t + u * step, f[u]);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) m = fmaxf(m, group_amax(f[u]));
+  }
+  for (; t < n16; t += step) {
+    float f[16];
+    src.load16(t, f);
     m = fmaxf(m, group_amax(f));
   }
 #pragma unroll
   for (int d = 32; d > 0; d >>= 1) m = fmaxf(m, __shfl_xor(m, d, 64));
-  if ((threadIdx.x & 63) == 0) atomicMax(out, __float_as_uint(m));
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int w = 1; w < 8; ++w) m = fmaxf(m, part[w]);
+    if (__float_as_uint(m) > __hip_atomic_load(out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMax(out, __float_as_uint(m));
+  }
+}
+
+template <class Src>
+static void launch_absmax(const Src& src, int64_t N, int K, float* out, hipStream_t st) {
+  const int64_t n16 = N * (K / 16);
+  const unsigned grid = (unsigned)std::min<int64_t>((n16 + 511) / 512, (int64_t)device_cus() * 2);
+  hipLaunchKernelGGL(absmax_kernel<Src>, dim3(grid), dim3(512), 0, st, src, n16, reinterpret_cast<uint32_t*>(out));
 }
 
 // The e4m3 INT2 target, one wave per row: the row scale R[row] =
@@ -387,10 +583,27 @@ static bool al(const void* p, int a) { return (reinterpret_cast<uintptr_t>(p) & 
 
 template <class Src, class Q>
 static int launch_q(const Src& src, const Q& q, int64_t N, int K, hipStream_t st) {
+  const int64_t n16 = N * (K / 16);
+  if (n16 == 0) return FP4X_OK;
+  hipLaunchKernelGGL((quant_kernel<Src, Q>), dim3((unsigned)((n16 + 255) / 256)), dim3(256), 0, st, src, q, n16);
+  return check_launch("quantize");
+}
+template <class Src, class Q>
+static int launch_q_groups(const Src& src, const Q& q, int64_t N, int K, hipStream_t st) {
   const int64_t groups = N * (K / Q::G);
   if (groups == 0) return FP4X_OK;
-  hipLaunchKernelGGL((quant_kernel<Src, Q>), dim3((unsigned)((groups + 255) / 256)), dim3(256), 0, st, src, q, N, K);
+  hipLaunchKernelGGL((quant_group_kernel<Src, Q>), dim3((unsigned)((groups + 255) / 256)), dim3(256), 0, st, src, q, N,
+                     K);
   return check_launch("quantize");
+}
+template <class Src>
+static int launch_nv4_amax(const Src& src, int64_t N, int K, float* amax, uint8_t* P, uint8_t* S, hipStream_t st) {
+  const int64_t n16 = N * (K / 16);
+  if (n16 == 0) return FP4X_OK;
+  launch_absmax(src, N, K, amax, st);
+  const unsigned grid = (unsigned)std::min<int64_t>((n16 + 255) / 256, (int64_t)device_cus() * 16);
+  hipLaunchKernelGGL(quant_nv4_amax_kernel<Src>, dim3(grid), dim3(256), 0, st, src, QNV4{P, S, 0.0f}, n16, amax);
+  return check_launch("quantize_nv4");
 }
 
 template <class Src>
@@ -400,8 +613,8 @@ static int dispatch_q(const Src& src, int64_t N, int K, int dst, int G, int qmax
     case FP4X_Q_W8:
       return launch_q(src, QW8{static_cast<int8_t*>(o0), static_cast<float*>(o1)}, N, K, st);
     case FP4X_Q_W6:
-      return launch_q(src, QW6{static_cast<uint8_t*>(o0), static_cast<uint8_t*>(o1), static_cast<uint16_t*>(o2), qmax},
-                      N, K, st);
+      return launch_q(
+          src, QW6{{static_cast<uint8_t*>(o0), static_cast<uint8_t*>(o1), static_cast<uint16_t*>(o2), qmax}}, N, K, st);
     case FP4X_Q_NV4:
       return launch_q(src, QNV4{static_cast<uint8_t*>(o0), static_cast<uint8_t*>(o1), gs}, N, K, st);
     case FP4X_Q_INT2_E4M3: {
@@ -498,13 +711,13 @@ int fp4x_quantize_w6_clip(int src, const void* src_a, const void* src_b, float s
   hipStream_t st = (hipStream_t)stream;
   switch (src) {
     case FP4X_SRC_F32:
-      return launch_q(SrcF32{static_cast<const float*>(src_a), K}, q, N, K, st);
+      return launch_q_groups(SrcF32{static_cast<const float*>(src_a), K}, q, N, K, st);
     case FP4X_SRC_BF16:
-      return launch_q(SrcBF16{static_cast<const uint16_t*>(src_a), K}, q, N, K, st);
+      return launch_q_groups(SrcBF16{static_cast<const uint16_t*>(src_a), K}, q, N, K, st);
     case FP4X_SRC_MX8:
-      return launch_q(SrcMX8{static_cast<const uint8_t*>(src_a), static_cast<const uint8_t*>(src_b), K}, q, N, K, st);
+      return launch_q_groups(SrcMX8{static_cast<const uint8_t*>(src_a), static_cast<const uint8_t*>(src_b), K}, q, N, K, st);
     default:
-      return launch_q(SrcNV4{static_cast<const uint8_t*>(src_a), static_cast<const uint8_t*>(src_b), src_gs, K}, q, N,
+      return launch_q_groups(SrcNV4{static_cast<const uint8_t*>(src_a), static_cast<const uint8_t*>(src_b), src_gs, K}, q, N,
                       K, st);
   }
 }
@@ -516,28 +729,40 @@ int fp4x_absmax(int src, const void* src_a, const void* src_b, float src_gs, int
   if (!out) { set_error("absmax: no output"); return FP4X_ERR_ARG; }
   if (N == 0) return FP4X_OK;
   hipStream_t st = (hipStream_t)stream;
-  const int64_t groups = N * (K / 16);
-  const unsigned grid = (unsigned)std::min<int64_t>((groups + 255) / 256, (int64_t)device_cus() * 8);
-  uint32_t* o = reinterpret_cast<uint32_t*>(out);
   switch (src) {
-    case FP4X_SRC_F32:
-      hipLaunchKernelGGL(absmax_kernel<SrcF32>, dim3(grid), dim3(256), 0, st, SrcF32{static_cast<const float*>(src_a), K},
-                         N, K, o);
-      break;
-    case FP4X_SRC_BF16:
-      hipLaunchKernelGGL(absmax_kernel<SrcBF16>, dim3(grid), dim3(256), 0, st,
-                         SrcBF16{static_cast<const uint16_t*>(src_a), K}, N, K, o);
-      break;
+    case FP4X_SRC_F32: launch_absmax(SrcF32{static_cast<const float*>(src_a), K}, N, K, out, st); break;
+    case FP4X_SRC_BF16: launch_absmax(SrcBF16{static_cast<const uint16_t*>(src_a), K}, N, K, out, st); break;
     case FP4X_SRC_MX8:
-      hipLaunchKernelGGL(absmax_kernel<SrcMX8>, dim3(grid), dim3(256), 0, st,
-                         SrcMX8{static_cast<const uint8_t*>(src_a), static_cast<const uint8_t*>(src_b), K}, N, K, o);
+      launch_absmax(SrcMX8{static_cast<const uint8_t*>(src_a), static_cast<const uint8_t*>(src_b), K}, N, K, out, st);
       break;
     default:
-      hipLaunchKernelGGL(absmax_kernel<SrcNV4>, dim3(grid), dim3(256), 0, st,
-                         SrcNV4{static_cast<const uint8_t*>(src_a), static_cast<const uint8_t*>(src_b), src_gs, K}, N,
-                         K, o);
+      launch_absmax(SrcNV4{static_cast<const uint8_t*>(src_a), static_cast<const uint8_t*>(src_b), src_gs, K}, N, K,
+                    out, st);
   }
   return check_launch("absmax");
+}
+
+int fp4x_quantize_nv4(int src, const void* src_a, const void* src_b, float src_gs, int64_t N, int K, float* amax,
+                      void* P, void* S, void* stream) {
+  int rc = src_check(src, src_a, src_b, N, K);
+  if (rc) return rc;
+  if (!al(P, 16) || !S || !amax) {
+    set_error("quantize_nv4: P must be 16-byte aligned, and S and amax given");
+    return FP4X_ERR_ARG;
+  }
+  hipStream_t st = (hipStream_t)stream;
+  uint8_t* p = static_cast<uint8_t*>(P);
+  uint8_t* s = static_cast<uint8_t*>(S);
+  switch (src) {
+    case FP4X_SRC_F32: return launch_nv4_amax(SrcF32{static_cast<const float*>(src_a), K}, N, K, amax, p, s, st);
+    case FP4X_SRC_BF16: return launch_nv4_amax(SrcBF16{static_cast<const uint16_t*>(src_a), K}, N, K, amax, p, s, st);
+    case FP4X_SRC_MX8:
+      return launch_nv4_amax(SrcMX8{static_cast<const uint8_t*>(src_a), static_cast<const uint8_t*>(src_b), K}, N, K,
+                             amax, p, s, st);
+    default:
+      return launch_nv4_amax(SrcNV4{static_cast<const uint8_t*>(src_a), static_cast<const uint8_t*>(src_b), src_gs, K},
+                             N, K, amax, p, s, st);
+  }
 }
 
 }  // extern "C"

@@ -610,15 +610,16 @@ def _hip_w6_clip(src, n, k, qmax, clip_search):
 
 
 def _hip_nv4(src, n, k):
-    """NVFP4 of a source: the global amax on the device (one host read, as the
-    reference's .item()), gs = max(amax / 6 / 448, 1e-30), then the groups."""
+    """NVFP4 of a source: the global amax, gs = max(amax / 6 / 448, 1e-30) and
+    the groups on the device, then one host read of amax for the returned gs
+    (the reference's .item())."""
     kind, a, b, sgs = src
     amax = torch.zeros(1, dtype=torch.float32, device=a.device)
-    _L.check(_L.lib().fp4x_absmax(kind, _ptr(a), None if b is None else _ptr(b), float(sgs), n, k, _ptr(amax),
-                                  _L.stream_of(a)), "absmax")
-    gs = max(float(amax.item()) / 6.0 / 448.0, 1e-30)
-    P, S = _hip_quantize(src, n, k, _Q_NV4, gs=gs)
-    return P, S, gs
+    P = torch.empty((n, k // 2), dtype=torch.uint8, device=a.device)
+    S = torch.empty((n, k // 16), dtype=torch.float8_e4m3fn, device=a.device)
+    _L.check(_L.lib().fp4x_quantize_nv4(kind, _ptr(a), None if b is None else _ptr(b), float(sgs), n, k, _ptr(amax),
+                                        _ptr(P), _ptr(S), _L.stream_of(a)), "quantize_nv4")
+    return P, S, max(float(amax.item()) / 6.0 / 448.0, 1e-30)
 
 
 def requantize_mx8(w8, s_u8, fmt, group=16, qmax=31, clip_search=0, scale_fmt="fp16"):

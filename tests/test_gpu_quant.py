@@ -205,3 +205,63 @@ def test_head_sized_int2_from_mx8(gpu, F):
     assert same(np_(P[rows]), Po) and same(np_(S[rows]), So)
     P, S, R = F.quantize_int2(wf, scale_fmt="e4m3", group=16)         # the row-scaled e4m3 form
     check("int2e", (P[rows], S[rows], R[rows]), wf[rows].cpu().numpy())
+
+
+def _boundary_rows(k=2560):
+    """fp32 rows whose quotients by the group scale lie on the code boundaries
+    and one or two fp32 steps to either side: halves of the W8 and W6 grids,
+    e2m1 midpoints, +-1 and 0 of the INT2 levels (group maxima fixed so that
+    the scales are not powers of two), with -0 and the smallest subnormals."""
+    rng = np.random.default_rng(77)
+    rows = []
+
+    def around(v):
+        v = np.asarray(v, np.float32)
+        step = rng.integers(-2, 3, v.shape)
+        for _ in range(2):
+            v = np.where(step > 0, np.nextafter(v, np.float32(np.inf)), np.where(step < 0, np.nextafter(v, -np.float32(np.inf)), v))
+            step = step - np.sign(step)
+        return v.astype(np.float32)
+
+    for scale in (0.0123, 0.7, 1.9, 2.6e-5):
+        a = np.float32(scale)
+        for half, top in ((127, 64), (31, 32)):
+            s = a / np.float32(half)
+            if half == 31:
+                s = np.float32(max(np.float32(np.float16(s)), np.float32(6.2e-5)))
+            r = around((rng.integers(-half, half, k) + 0.5).astype(np.float32) * s)
+            r = np.clip(r, -a, a)
+            r[::top] = a
+            rows.append(r)
+        gs = np.float32(1e-4)
+        for _ in range(2):
+            sf = np.float32(2.0 ** int(rng.integers(-3, 4))) * np.float32(1 + int(rng.integers(0, 8)) / 8) * gs
+            mids = np.array([.25, .75, 1.25, 1.75, 2.5, 3.5, 5.0], np.float32)
+            r = around(rng.choice(mids, k) * sf) * rng.choice(np.array([-1, 1], np.float32), k)
+            r[::16] = np.float32(6) * sf
+            rows.append(r.astype(np.float32))
+        s = np.float32(np.float16(a / np.float32(1.5)))
+        r = around(rng.choice(np.array([-1, 1, 0], np.float32), k) * s)
+        r[5::7] = -0.0
+        r[6::11] = np.float32(-1e-45)
+        r[::16] = a
+        rows.append(r)
+    return np.stack(rows).astype(np.float32)
+
+
+@pytest.mark.parametrize("fmt", ["w8", "w6", "nv4", "int2"])
+def test_code_boundaries(gpu, F, fmt):
+    """Codes taken without a division equal the divided ones on and beside
+    every boundary, also with a global NVFP4 scale above and below it."""
+    w = _boundary_rows()
+    t = dev(w)
+    if fmt == "int2":
+        for grp in (16, 32, 64):
+            check(fmt, F.quantize_int2(t, group=grp), w, group=grp)
+    elif fmt == "nv4":
+        for peak in (0.0, 0.27, 40.0):
+            w2 = w.copy()
+            w2[0, 0] = max(w2[0, 0], np.float32(peak))
+            check(fmt, F.quantize_nv4(dev(w2)), w2)
+    else:
+        check(fmt, F.quantize_w8(t) if fmt == "w8" else F.quantize_w6(t), w)
