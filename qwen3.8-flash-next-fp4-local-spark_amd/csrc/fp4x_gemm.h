@@ -22,9 +22,10 @@
 // its loads alone take 17 of 19 us and grow by 1.9 us per 16 rows, which is
 // the tile's bytes (weights from HBM, activations from L2) at about 40 GB/s
 // per CU, whatever the ring's depth; loads that all hit L2 reach 140.  So
-// tiles are as large as leaves every CU one, and M = 256 (26 us of loads, 30
-// of decoding and MFMA, 38 in all) would gain from a better overlap of the
-// two.
+// tiles are as large as leaves every CU one.  At M = 256 (26 us of loads, 30
+// of decoding and MFMA, 38-40 in all) larger wave tiles, through direct loads
+// or registers, took 37-41 and were slower on every narrower matrix; torch's
+// bf16 product of that size takes 41 with its weights from HBM.
 //
 // us per call, graph replays from HBM, one launch per 16 rows -> this:
 //   M                     24          64          256
