@@ -120,21 +120,24 @@ constexpr int kGemmKB = 128;                       // k values of a unit
 // Scales: 16 rows x 2 dwords that hold the row's scales of the unit, the
 // first one at byte `off & 3` where the rows' scales are only 2-byte aligned.
 struct GemmScales {
-  const uint8_t* s;
+  const uint8_t* s;                                // a whole dword of the plane
   uint32_t o;                                      // this lane's row's scale bytes, from s
-  int last;                                        // last dword of the plane, from s
-  // rb: scale bytes of a row
-  __device__ void set(const uint8_t* plane, int64_t n0, int row, int rb, int64_t N) {
-    s = plane + ((n0 * rb) & ~(int64_t)3);
-    o = (uint32_t)(row * rb + (int)((n0 * rb) & 3));
-    const int64_t left = (N - n0) * rb + ((n0 * rb) & 3) - 4;
-    last = (int)(left < 0x7ffffffc ? left : 0x7ffffffc) & ~3;
+  int last;                                        // last whole dword of the plane, from s
+  // rb: scale bytes of a row; the plane holds at least one whole dword.  A
+  // strip of the last row alone can begin past the last whole dword (two bytes
+  // a row, K = 64, N odd): s is then that dword, so no offset is below 0.
+  __host__ __device__ void set(const uint8_t* plane, int64_t n0, int row, int rb, int64_t N) {
+    const int64_t at = n0 * rb, end = N * rb - 4, b = (at < end ? at : end) & ~(int64_t)3;
+    s = plane + b;
+    o = (uint32_t)(row * rb + (int)(at - b));
+    last = (int)(end - b < 0x7ffffffc ? end - b : 0x7ffffffc) & ~3;
   }
   // ub: scale bytes of a row in a unit; d: dword 0 or 1
-  __device__ void issue(char* l, int ku, int ub, int d) const {
-    const int at = (int)((o + ku * ub) & ~3u) + 4 * d;
-    dma_b32(s + (uint32_t)(at < last ? at : last), l);
+  __host__ __device__ const uint8_t* at(int ku, int ub, int d) const {
+    const int a = (int)((o + ku * ub) & ~3u) + 4 * d;
+    return s + (uint32_t)(a < last ? a : last);
   }
+  __device__ void issue(char* l, int ku, int ub, int d) const { dma_b32(at(ku, ub, d), l); }
 };
 
 template <class F> struct GemmUnit;

@@ -79,6 +79,18 @@ def test_gemm_up_to_16_rows(gpu, F, fmt, M, N, K, monkeypatch):
         check(F, fmt, planes, w_op, gs, x, bf16_dev(x))
 
 
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("M,N", [(17, 17), (40, 33), (130, 4099), (33, 2)])
+def test_gemm_one_unit_rows(gpu, F, fmt, M, N):
+    """K = 64: rows of half a unit and, for MXFP8 and fp16 W8 scales, of two
+    scale bytes, so that with N odd the last row begins past the scale plane's
+    last whole dword (where the loads go is checked in test_gemm_scales.py)."""
+    rng = np.random.default_rng(M + N)
+    planes, w_op, gs = planes_of(fmt, rng, N, 64)
+    x, _ = act(rng, M, 64)
+    check(F, fmt, planes, w_op, gs, x, bf16_dev(x))
+
+
 def test_gemm_bf16_short_tail(gpu, F):
     """K a multiple of 16 only (bf16)."""
     rng = np.random.default_rng(5)
