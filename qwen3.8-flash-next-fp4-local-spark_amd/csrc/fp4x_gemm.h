@@ -865,9 +865,15 @@ bool launch_gemm_cfg(const GemvLaunch& p, hipStream_t st) {
   static_assert(S::XI * C::WN == 4 * C::MT, "activation loads divide over the waves");
   auto kern = gemm_kernel<F, C::MT, C::NT, C::WN, C::WK, C::D>;
   if constexpr (S::LDS > 64 * 1024) {
-    static const bool ok = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, S::LDS) == hipSuccess;
-    if (!ok) return false;
+    static bool attr_set = false;
+    if (!attr_set) {
+      if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              S::LDS) != hipSuccess) {
+        (void)hipGetLastError();                           // not the next launch's error
+        return false;
+      }
+      attr_set = true;
+    }
   }
   const int mtiles = (p.M + S::BM - 1) / S::BM, ntiles = (p.N + S::BN - 1) / S::BN;
   const int total = mtiles * ntiles, grid = (total + 7) / 8 * 8;
