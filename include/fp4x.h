@@ -338,7 +338,9 @@ int fp4x_hold_cus(int wgs, int64_t microseconds, int lds_kb, uint32_t* sink, voi
  * FP4X_NV4_STREAM, FP4X_W6_STREAM, FP4X_MX8_STREAM and FP4X_HC_MIX ("0"
  * selects the MFMA core or the two-call mixer), FP4X_HC_XCD ("0": the
  * single-launch mixer's down partials device-coherent rather than in one
- * XCD's L2), FP4X_ROWS, FP4X_WAVES_PER_CU, FP4X_HC_SPIN_LIMIT.  Not
+ * XCD's L2), FP4X_ROWS ("0": no few-rows kernels), FP4X_GEMM ("0": no
+ * blocked GEMM; FP4X_ROWS=0 and a format's stream switch turn it off too),
+ * FP4X_WAVES_PER_CU, FP4X_HC_SPIN_LIMIT.  Not
  * thread-safe against concurrent launches.  No counterpart in the reference
  * (its Triton launches take no such switches). */
 int fp4x_reload_env(void);

@@ -191,6 +191,7 @@ struct GemmRows64 {
 };
 
 template <> struct GemmUnit<FmtMX8> {
+  static bool on(const Switches& w) { return w.mx8_stream; }
   static constexpr int BYTES = 2048 + 128, NDMA = 3;
   static constexpr float DEQ = 0.5f;                // VALU operations per weight
   static constexpr int KMULT = 64;
@@ -271,6 +272,7 @@ template <> struct GemmUnit<FmtMX8> {
 };
 
 template <bool F16S> struct GemmUnit<FmtW8<F16S>> {
+  static bool on(const Switches& w) { return w.w8_stream; }
   static constexpr int BYTES = 2048 + 128, NDMA = 3, SB = F16S ? 2 : 4;
   static constexpr float DEQ = 2.5f;
   static constexpr int KMULT = 64;
@@ -389,6 +391,7 @@ template <bool F16S> struct GemmUnit<FmtW8<F16S>> {
 };
 
 template <> struct GemmUnit<FmtW6> {
+  static bool on(const Switches& w) { return w.w6_stream; }
   static constexpr int BYTES = 1024 + 512 + 128, NDMA = 3;
   static constexpr float DEQ = 3.9f;                // VALU operations per weight
   static constexpr int KMULT = 64;
@@ -473,6 +476,7 @@ template <> struct GemmUnit<FmtW6> {
 };
 
 template <> struct GemmUnit<FmtNV4> {
+  static bool on(const Switches& w) { return w.nv4_stream; }
   static constexpr int BYTES = 1024 + 128, NDMA = 2;
   static constexpr float DEQ = 2.0f;                // VALU operations per weight
   static constexpr int KMULT = 64;
@@ -539,6 +543,7 @@ template <> struct GemmUnit<FmtNV4> {
 };
 
 template <> struct GemmUnit<FmtBF16> {
+  static bool on(const Switches&) { return true; }
   static constexpr int BYTES = 4096, NDMA = 4;
   static constexpr float DEQ = 0.0f;                // VALU operations per weight
   static constexpr int KMULT = 16;
@@ -931,11 +936,11 @@ GemmChoice gemm_choose(const GemvLaunch& p, int cus) {
 // start (its last two bytes apart).  False, and nothing launched, otherwise.
 template <class F>
 bool launch_gemm(const GemvLaunch& p, hipStream_t st) {
-  if (!switches().gemm || p.M < 1 || p.N < 1) return false;
+  // a switch that sends the format's calls to the core turns this kernel off too
+  const Switches& sw = switches();
+  if (!sw.gemm || !sw.rows || !GemmUnit<F>::on(sw) || p.M < 1 || p.N < 1) return false;
   auto al = [](const void* q, int n) { return (reinterpret_cast<uintptr_t>(q) & (uintptr_t)(n - 1)) == 0; };
   const int K = p.pa.K;
-  // FP4X_ROWS=0 sends matrices of few rows to the core
-  if (p.M <= 16 && !switches().rows && (p.N + 15) / 16 * 2 < device_cus()) return false;
   if (!al(p.x, 16) || p.x_stride % 8 || !al(p.pa.w0, 16)) return false;
   if (K > 1 << 20 || p.x_stride > 1 << 23) return false;
   if (GemmUnit<F>::KMULT > 16 && K % GemmUnit<F>::KMULT) return false;

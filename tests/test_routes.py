@@ -1,0 +1,37 @@
+"""Which kernel a dense linear launches, without a GPU (tests/standin.py, 256
+CUs): the path switches."""
+import pytest
+
+import standin
+
+
+@pytest.fixture(scope="module")
+def route(tmp_path_factory):
+    if not standin.available():
+        pytest.skip("no g++ or no library")
+    so = standin.build(tmp_path_factory.mktemp("standin"))
+    return lambda code, **env: standin.run(so, code, **env)
+
+
+def test_switches_that_force_the_core(route):
+    """FP4X_ROWS=0 and a format's stream switch send its calls to the MFMA core
+    also where the blocked GEMM would take them, for any number of rows."""
+    route(r"""
+STREAM = {"mx8": "FP4X_MX8_STREAM", "w8": "FP4X_W8_STREAM", "w8_f16": "FP4X_W8_STREAM", "w6": "FP4X_W6_STREAM",
+          "nv4": "FP4X_NV4_STREAM"}
+for fmt in FMT:
+    for M, N, K in ((16, 8300, 1984), (6, 5000, 1920), (13, 1600, 1088), (24, 512, 2560), (256, 16384, 2560)):
+        call = linear if M <= 16 else rows
+        rc, names = call(fmt, M, N, K)
+        assert rc == B.OK and "gemm_kernel" in names[0], (fmt, M, N, K, names)
+        for env in ("FP4X_GEMM", "FP4X_ROWS", STREAM.get(fmt)):
+            if env is None:
+                continue
+            switches(**{env: "0"})
+            rc, names = call(fmt, M, N, K)
+            switches(**{env: None})
+            if M > 16:
+                assert rc == B.NOT_TAKEN and not names, (fmt, M, N, K, env, names)
+            else:
+                assert rc == B.OK and "gemv_mfma_kernel" in names[0], (fmt, M, N, K, env, names)
+""")
