@@ -154,3 +154,22 @@ def test_gemm_graph(gpu, F):
         torch.cuda.synchronize()
         assert torch.equal(y, want)
         assert torch.equal(run(F, "w6", x, planes, 1), want)
+
+
+@pytest.mark.parametrize("fmt", ["mx8", "w8", "w6", "nv4", "bf16"])
+@pytest.mark.parametrize("K,bk,ks", [(512, 8, 64), (8320, 64, 130), (8320, 64, 65)])
+def test_gemm_refuses_bad_k_splits(gpu, F, fmt, K, bk, ks):
+    """K splits that 16 rows refuse (slices that are no whole chunks, or more
+    than 64 of them) are refused for more rows too; a good one is accepted."""
+    rng = np.random.default_rng(ks)
+    planes, _, _ = planes_of(fmt, rng, 32, K)
+    x = bf16_dev(act(rng, 20, K)[0])
+
+    def call(m, bk, ks):
+        cfg = (32, bk, 4, ks) if fmt == "nv4" else (32, bk, ks, 4)
+        fn = {"mx8": F.mx8_linear, "w8": F.w8_linear, "w6": F.w6_linear, "nv4": F.nv4_linear, "bf16": F.bf16_linear}[fmt]
+        return fn(x[:m], *planes, cfg)
+    for m in (16, 20):
+        with pytest.raises(ValueError):
+            call(m, bk, ks)
+    assert call(20, 32, 2).shape == (20, 32)
