@@ -114,8 +114,9 @@ int fp4x_nv4_linear(const void* x, int64_t x_stride, const void* P, const void* 
  * The K sum of an output is split by the kernel, in a fixed order.  Returns
  * FP4X_NOT_TAKEN, with nothing launched, for what only the entry points of up
  * to 16 rows take (K not a multiple of 64 but for BF16, a scale plane not
- * 4-byte aligned, W6's H not 16-byte aligned, K > 2^20, x_stride > 2^23): call
- * those per 16 rows.
+ * 4-byte aligned or of under 4 bytes, W6's H not 16-byte aligned, K > 2^20,
+ * x_stride > 2^23), where the path switches turn the kernel off, and where the
+ * runtime refuses its LDS: call those per 16 rows.
  * [the same functions, x/fp4x_kernels.py:50-70, :102-113, :147-148, :270-271] */
 int fp4x_linear_rows(int fmt, const void* x, int64_t x_stride, const void* w0, const void* w1, const void* s, float gs,
                      void* out, int out_dtype, int M, int N, int K, void* stream);

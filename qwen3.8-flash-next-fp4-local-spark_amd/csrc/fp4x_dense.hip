@@ -338,6 +338,8 @@ int fp4x_linear_rows(int fmt, const void* x, int64_t x_stride, const void* w0, c
   if (rc) return rc;
   if (!aligned(w0, 16)) return fail(FP4X_ERR_ARG, "linear_rows: weight rows must be 16-byte aligned");
   if (M == 0 || N == 0) return FP4X_OK;
+  if ((fmt != FP4X_FMT_BF16 && !s) || (fmt == FP4X_FMT_W6 && !w1))
+    return fail(FP4X_ERR_ARG, "linear_rows: the format's scales (and W6's bit-pair plane) must be given");
   GemvLaunch p = base_launch(fmt, x, x_stride, out, out_dtype, N, M, N, K, 1, nullptr, nullptr);
   p.pa.w0 = static_cast<const uint8_t*>(w0);
   p.pa.w1 = fmt == FP4X_FMT_W6 ? static_cast<const uint8_t*>(w1) : nullptr;

@@ -29,7 +29,7 @@ def test_header_declares_entry_points():
                  "fp4x_topk_rows", "fp4x_refine_mx8", "fp4x_hc_down", "fp4x_hc_up", "fp4x_hc_scaled_silu",
                  "fp4x_hc_gate_mean", "fp4x_bf16_linear", "fp4x_w8_linear_layers", "fp4x_mx8_dequant",
                  "fp4x_hc_mix", "fp4x_int2_topk", "fp4x_refine_nv4", "fp4x_scatter_draft", "fp4x_quantize",
-                 "fp4x_absmax", "fp4x_draft_nv4"):
+                 "fp4x_absmax", "fp4x_draft_nv4", "fp4x_linear_rows", "fp4x_quantize_nv4"):
         assert must in names
 
 
@@ -106,6 +106,36 @@ def test_argument_errors_without_gpu(lib):
     assert b"bad target" in L.fp4x_last_error()
     assert Q(2, None, None, 0.0, 8, 128, 0, 16, 31, 0.0, None, None, None, None) == _fp4x.ERR_ARG
     assert L.fp4x_absmax(1, None, None, 0.0, 8, 100, None, None) == _fp4x.ERR_ARG
+    # the linears of any number of rows: formats it does not have, K off the format's multiple, misaligned planes
+    # or activations, and planes that the format needs
+    R, A = L.fp4x_linear_rows, ctypes.c_void_p(1 << 40)              # never read: nothing runs
+    for fmt in (-1, _fp4x.FMT_INT2_F16, _fp4x.FMT_INT2_E4M3, 8):
+        assert R(fmt, A, 2560, A, None, A, 1.0, A, 0, 24, 64, 2560, None) == _fp4x.ERR_ARG
+    assert b"weight format" in L.fp4x_last_error()
+    assert R(_fp4x.FMT_W8_F32, A, 128, A, None, A, 1.0, A, 0, 24, 64, 96, None) == _fp4x.ERR_ARG
+    assert R(_fp4x.FMT_MX8, A, 2560, ctypes.c_void_p((1 << 40) + 8), None, A, 1.0, A, 0, 24, 64, 2560,
+             None) == _fp4x.ERR_ARG
+    assert b"16-byte aligned" in L.fp4x_last_error()
+    assert R(_fp4x.FMT_MX8, A, 2552, A, None, A, 1.0, A, 0, 24, 64, 2560, None) == _fp4x.ERR_ARG   # stride < K
+    assert R(_fp4x.FMT_MX8, A, 2560, A, None, None, 1.0, A, 0, 24, 64, 2560, None) == _fp4x.ERR_ARG
+    assert R(_fp4x.FMT_W6, A, 2560, A, None, A, 1.0, A, 0, 24, 64, 2560, None) == _fp4x.ERR_ARG
+    assert b"must be given" in L.fp4x_last_error()
+    # what only the entries of up to 16 rows take is left to them: K off 64, scales off 4 bytes, W6's H off 16
+    assert R(_fp4x.FMT_NV4, A, 96, A, None, A, 1.0, A, 0, 24, 64, 96, None) == _fp4x.NOT_TAKEN
+    assert R(_fp4x.FMT_NV4, A, 128, A, None, ctypes.c_void_p((1 << 40) + 2), 1.0, A, 0, 24, 64, 128,
+             None) == _fp4x.NOT_TAKEN
+    assert R(_fp4x.FMT_W6, A, 128, A, ctypes.c_void_p((1 << 40) + 8), A, 1.0, A, 0, 24, 64, 128,
+             None) == _fp4x.NOT_TAKEN
+    assert R(_fp4x.FMT_MX8, None, 2560, None, None, None, 1.0, None, 0, 0, 64, 2560, None) == _fp4x.OK
+    # NVFP4 quantization in one call: K % 64, an unknown source, packed sources without scales, missing outputs
+    V = L.fp4x_quantize_nv4
+    assert V(0, A, None, 0.0, 8, 96, A, A, A, None) == _fp4x.ERR_ARG
+    assert V(4, A, None, 0.0, 8, 128, A, A, A, None) == _fp4x.ERR_ARG
+    assert V(2, A, None, 0.0, 8, 128, A, A, A, None) == _fp4x.ERR_ARG
+    assert V(0, A, None, 0.0, 8, 128, None, A, A, None) == _fp4x.ERR_ARG
+    assert V(0, A, None, 0.0, 8, 128, A, A, None, None) == _fp4x.ERR_ARG
+    assert b"quantize_nv4" in L.fp4x_last_error()
+    assert V(0, A, None, 0.0, 0, 128, A, A, A, None) == _fp4x.OK
     # the CU-holding test kernel: bounded time and LDS
     assert L.fp4x_hold_cus(8, 200000, 160, None, None) == _fp4x.ERR_ARG
     assert L.fp4x_hold_cus(8, 100, 161, None, None) == _fp4x.ERR_ARG
