@@ -264,9 +264,12 @@ int fp4x_w8_linear_layers(const void* x, int64_t x_stride, int64_t x_lstride, co
   // through LDS; other single matrices without split-K take the blocked GEMM,
   // and the rest the MFMA core
   hipStream_t st = (hipStream_t)stream;
-  // the mixer's up projection (rows much shorter than they are many) stays on
-  // the core, whose sums the single-launch mixer reproduces bit for bit
-  const bool one = layers == 1 && ksplit == 1 && !(K <= 1024 && N >= 8 * K);
+  // the mixer's up projection [4 H x lr] stays on the core, whose sums hc_up
+  // and the single-launch mixer reproduce bit for bit: up to lr = 1024 and from
+  // H = 1.5 lr on (the served shape has H = 8 lr).  That equality costs other
+  // matrices of such a shape the GEMM's time: [4096 x 640] at M = 5 / 16 takes
+  // 6.2 / 7.4 us on the core and 4.6 / 4.6 in the GEMM
+  const bool one = layers == 1 && ksplit == 1 && !(K <= 1024 && N >= 6 * (int64_t)K);
   if (fmt == FP4X_FMT_W8_F16) {
     if (launch_w8_stream<true>(p, layers, st)) return check_launch("w8_stream");
     if (layers == 1 && launch_w8_ktile<true, EpiStore>(p, st)) return check_launch("w8_ktile");

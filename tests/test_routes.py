@@ -1,5 +1,5 @@
 """Which kernel a dense linear launches, without a GPU (tests/standin.py, 256
-CUs): the path switches."""
+CUs): the path switches, and the mixer's up projection."""
 import pytest
 
 import standin
@@ -34,4 +34,19 @@ for fmt in FMT:
                 assert rc == B.NOT_TAKEN and not names, (fmt, M, N, K, env, names)
             else:
                 assert rc == B.OK and "gemv_mfma_kernel" in names[0], (fmt, M, N, K, env, names)
+""")
+
+
+def test_mixer_up_projection_stays_on_the_core(route):
+    """[4 H x lr] through w8_linear at 5 to 16 rows, which streams only where lr
+    is a multiple of 512: on the MFMA core, whose sums hc_up reproduces, over
+    hidden widths and ranks as far apart as H = 1.6 lr."""
+    route(r"""
+for h in range(1024, 2817, 64):
+    for lr in range(192, 641, 64):
+        for M in (5, 16):
+            for fmt in ("w8", "w8_f16"):
+                rc, names = linear(fmt, M, 4 * h, lr)
+                assert rc == B.OK and "gemm_kernel" not in names[0], (h, lr, M, fmt, names)
+                assert "gemv_mfma_kernel" in names[0] or lr % 512 == 0, (h, lr, M, fmt, names)
 """)
