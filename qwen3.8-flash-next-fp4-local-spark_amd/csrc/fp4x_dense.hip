@@ -32,7 +32,8 @@ bool launch_gemm_w8_f16(const GemvLaunch& p, hipStream_t st);
 bool launch_gemm_w6(const GemvLaunch& p, hipStream_t st);
 bool launch_gemm_nv4(const GemvLaunch& p, hipStream_t st);
 bool launch_gemm_bf16(const GemvLaunch& p, hipStream_t st);
-bool gemm_few_rows(const GemvLaunch& p);
+bool gemm_few_rows(const GemvLaunch& p, int fmt);
+bool gemm_few_tiles(const GemvLaunch& p);
 bool launch_w8_single_stream_f16(GemvLaunch p, hipStream_t st);
 bool launch_w8_single_stream_f32(GemvLaunch p, hipStream_t st);
 int topk_check(const void* logits, int dtype, int64_t stride, int M, int V, int C, void* workspace,
@@ -216,10 +217,9 @@ int fp4x_mx8_linear(const void* x, int64_t x_stride, const void* w, const void* 
   p.pa.s = static_cast<const uint8_t*>(s);
   if (launch_rows_wide<FmtMX8>(p, (hipStream_t)stream)) return check_launch("mx8_rows");    // 16-20 rows per CU, M = 1
   if (launch_mx8_stream_entry(p, (hipStream_t)stream)) return check_launch("mx8_stream");   // many tiles
-  if (gemm_few_rows(p) && launch_gemm_mx8(p, (hipStream_t)stream)) return check_launch("mx8_gemm");  // M > 8
   if (launch_rows_gemv<FmtMX8>(p, 1, (hipStream_t)stream)) return check_launch("mx8_rows");  // fewer rows
   if (launch_mx8_stream_tile_entry(p, (hipStream_t)stream)) return check_launch("mx8_stream"); // 1/2-1 tile per CU
-  if (ksplit == 1 && launch_gemm_mx8(p, (hipStream_t)stream)) return check_launch("mx8_gemm");
+  if ((ksplit == 1 || gemm_few_tiles(p)) && launch_gemm_mx8(p, (hipStream_t)stream)) return check_launch("mx8_gemm");
   return launch_gemv_mfma<FmtMX8, EpiStore>(p, 1, (hipStream_t)stream);
 }
 
@@ -231,9 +231,8 @@ int fp4x_bf16_linear(const void* x, int64_t x_stride, const void* w, void* out, 
   if (M == 0 || N == 0) return FP4X_OK;
   GemvLaunch p = base_launch(FP4X_FMT_BF16, x, x_stride, out, out_dtype, N, M, N, K, ksplit, part, tickets);
   p.pa.w0 = static_cast<const uint8_t*>(w);
-  if (gemm_few_rows(p) && launch_gemm_bf16(p, (hipStream_t)stream)) return check_launch("bf16_gemm");  // M > 8
   if (launch_rows_gemv<FmtBF16>(p, 1, (hipStream_t)stream)) return check_launch("bf16_rows");
-  if (ksplit == 1 && launch_gemm_bf16(p, (hipStream_t)stream)) return check_launch("bf16_gemm");
+  if ((ksplit == 1 || gemm_few_tiles(p)) && launch_gemm_bf16(p, (hipStream_t)stream)) return check_launch("bf16_gemm");
   return launch_gemv_mfma<FmtBF16, EpiStore>(p, 1, (hipStream_t)stream);
 }
 
@@ -273,7 +272,7 @@ int fp4x_w8_linear_layers(const void* x, int64_t x_stride, int64_t x_lstride, co
   if (fmt == FP4X_FMT_W8_F16) {
     if (launch_w8_stream<true>(p, layers, st)) return check_launch("w8_stream");
     if (layers == 1 && launch_w8_ktile<true, EpiStore>(p, st)) return check_launch("w8_ktile");
-    if (one && gemm_few_rows(p) && launch_gemm_w8_f16(p, st)) return check_launch("w8_gemm");
+    if (one && gemm_few_rows(p, fmt) && launch_gemm_w8_f16(p, st)) return check_launch("w8_gemm");
     if (launch_rows_gemv<FmtW8<true>>(p, layers, st)) return check_launch("w8_rows");   // few rows (a router gate)
     if (layers == 1 && launch_w8_single_stream_f16(p, st)) return check_launch("w8_single_stream");
     if (one && launch_gemm_w8_f16(p, st)) return check_launch("w8_gemm");
@@ -281,7 +280,7 @@ int fp4x_w8_linear_layers(const void* x, int64_t x_stride, int64_t x_lstride, co
   }
   if (launch_w8_stream<false>(p, layers, st)) return check_launch("w8_stream");
   if (layers == 1 && launch_w8_ktile<false, EpiStore>(p, st)) return check_launch("w8_ktile");
-  if (one && gemm_few_rows(p) && launch_gemm_w8_f32(p, st)) return check_launch("w8_gemm");
+  if (one && gemm_few_rows(p, fmt) && launch_gemm_w8_f32(p, st)) return check_launch("w8_gemm");
   if (launch_rows_gemv<FmtW8<false>>(p, layers, st)) return check_launch("w8_rows");
   if (layers == 1 && launch_w8_single_stream_f32(p, st)) return check_launch("w8_single_stream");
   if (one && launch_gemm_w8_f32(p, st)) return check_launch("w8_gemm");
@@ -306,11 +305,11 @@ int fp4x_w6_linear(const void* x, int64_t x_stride, const void* L, const void* H
   p.pa.s = static_cast<const uint8_t*>(S);
   if (launch_rows_wide<FmtW6>(p, (hipStream_t)stream)) return check_launch("w6_rows");       // many rows, M = 1
   if (launch_w6_stream_entry(p, (hipStream_t)stream)) return check_launch("w6_stream");     // many tiles
-  if (gemm_few_rows(p) && launch_gemm_w6(p, (hipStream_t)stream)) return check_launch("w6_gemm");  // M > 8
+  if (gemm_few_rows(p, FP4X_FMT_W6) && launch_gemm_w6(p, (hipStream_t)stream)) return check_launch("w6_gemm");
   if (launch_rows_gemv<FmtW6>(p, 1, (hipStream_t)stream)) return check_launch("w6_rows");    // fewer rows
   if (launch_w6_stream_one_entry(p, (hipStream_t)stream)) return check_launch("w6_stream");  // 1-2 tiles per CU
   if (launch_w6_stream_tile_entry(p, (hipStream_t)stream)) return check_launch("w6_stream"); // 1/2-1 tile per CU
-  if (ksplit == 1 && launch_gemm_w6(p, (hipStream_t)stream)) return check_launch("w6_gemm");
+  if ((ksplit == 1 || gemm_few_tiles(p)) && launch_gemm_w6(p, (hipStream_t)stream)) return check_launch("w6_gemm");
   return launch_gemv_mfma<FmtW6, EpiStore>(p, 1, (hipStream_t)stream);
 }
 
@@ -325,11 +324,11 @@ int fp4x_nv4_linear(const void* x, int64_t x_stride, const void* P, const void* 
   p.pa.s = static_cast<const uint8_t*>(S);
   p.gs = gs;
   if (launch_nv4_stream_entry(p, (hipStream_t)stream)) return check_launch("nv4_stream");   // many tiles
-  if (gemm_few_rows(p) && launch_gemm_nv4(p, (hipStream_t)stream)) return check_launch("nv4_gemm");  // M > 8
+  if (gemm_few_rows(p, FP4X_FMT_NV4) && launch_gemm_nv4(p, (hipStream_t)stream)) return check_launch("nv4_gemm");
   if (launch_rows_gemv<FmtNV4>(p, 1, (hipStream_t)stream)) return check_launch("nv4_rows");  // fewer rows
   if (launch_nv4_stream_one_entry(p, (hipStream_t)stream)) return check_launch("nv4_stream"); // 1-2 tiles per CU
   if (launch_nv4_stream_tile_entry(p, (hipStream_t)stream)) return check_launch("nv4_stream"); // 1/2-1 tile per CU
-  if (ksplit == 1 && launch_gemm_nv4(p, (hipStream_t)stream)) return check_launch("nv4_gemm");
+  if ((ksplit == 1 || gemm_few_tiles(p)) && launch_gemm_nv4(p, (hipStream_t)stream)) return check_launch("nv4_gemm");
   return launch_gemv_mfma<FmtNV4, EpiStore>(p, 1, (hipStream_t)stream);
 }
 

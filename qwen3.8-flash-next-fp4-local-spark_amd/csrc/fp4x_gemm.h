@@ -40,6 +40,7 @@
 #pragma once
 #include <type_traits>
 #include "fp4x_stream.h"
+#include "../../include/fp4x.h"
 
 namespace fp4x {
 
@@ -955,14 +956,36 @@ bool launch_gemm(const GemvLaunch& p, hipStream_t st) {
   return c.fn(p, st);
 }
 
-// Matrices of few rows (the few-rows kernels' shapes) at M > 8: this kernel
-// instead, but for short rows up to M = 12.  us, few-rows kernel -> this, at M
-// = 8 / 12 / 16: MXFP8 [512 x 2560] 4.1 -> 4.4 / 5.0 -> 4.6 / 5.4 -> 4.7, W6
-// 4.2 -> 5.0 / 5.1 -> 5.1 / 5.5 -> 5.3, NVFP4 [96 x 2560] 3.8 -> 3.9 / 4.7 ->
-// 3.9 / 5.1 -> 3.9; W8 [900 x 1088] 3.5 -> 4.1 / 3.9 -> 4.0 / 4.1 -> 4.0.
-inline bool gemm_before_rows(const GemvLaunch& p) {
+// Matrices under half a tile per CU that the few-rows kernels leave (over 4
+// rows per CU, or rows too long for them): this kernel rather than the core at
+// M > 8, but for short rows at M > 12, also for calls with a K split.
+inline bool gemm_small(const GemvLaunch& p) {
   const int tiles = (p.N + 15) / 16;
   return tiles * 2 < device_cus() && p.M > (p.pa.K < 2048 ? 12 : 8) && (p.ksplit == 1 || p.pa.K <= 4096);
+}
+
+// Those of the few-rows kernels' shapes that this kernel takes first.  us with
+// weights from HBM (64 matrices, 1 GB written before each replay), few-rows
+// kernel / this, [512 x K]:
+//   K               M = 13, 1088   2560         4096         6144
+//   NVFP4           5.13 / 4.41    6.02 / 5.53  7.20 / 6.92  8.88 / 8.77
+//   W6              5.22 / 4.81    6.17 / 6.50  7.48 / 7.77  9.26 / 10.00
+//   MXFP8           4.85 / 4.85    5.95 / 5.95  7.19 / 7.67  8.99 / 9.74
+//   bf16            4.88 / 4.95    6.09 / 6.51  7.32 / 7.86  9.06 / 10.11
+// NVFP4 at M = 9: 2560 5.63 / 5.27, 4096 6.55 / 6.92, 6144 7.95 / 8.72; the
+// other formats lose up to a quarter there.  W8 stands between W6 and MXFP8
+// (M = 13: 0.93-1.02 of the few-rows time below K = 2048, 1.01-1.08 beyond).
+// N from 48 to 1016 moves none of these by more than a few percent.  MXFP8
+// and bf16 are at 0.95-1.05 at best (M = 16), so their few-rows kernel stays.
+inline bool gemm_before_rows(const GemvLaunch& p, int fmt) {
+  if (!gemm_small(p)) return false;
+  switch (fmt) {
+    case FP4X_FMT_NV4: return p.pa.K < 4096 || p.M > 12;
+    case FP4X_FMT_W6:
+    case FP4X_FMT_W8_F32:
+    case FP4X_FMT_W8_F16: return p.pa.K < 2048;
+    default: return false;
+  }
 }
 
 }  // namespace fp4x

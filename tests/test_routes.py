@@ -50,3 +50,31 @@ for h in range(1024, 2817, 64):
                 assert rc == B.OK and "gemm_kernel" not in names[0], (h, lr, M, fmt, names)
                 assert "gemv_mfma_kernel" in names[0] or lr % 512 == 0, (h, lr, M, fmt, names)
 """)
+
+
+def test_few_rows_lines(route):
+    """Matrices of few rows at 9 to 16 activation rows, on either side of the
+    lines between the few-rows kernels and the blocked GEMM (measured beside
+    gemm_before_rows); over 4 rows per CU, and rows too long for the few-rows
+    kernels, the GEMM takes all of them."""
+    route(r"""
+def gemm(fmt, M, N, K, ks=1):
+    rc, names = linear(fmt, M, N, K, ks)
+    assert rc == B.OK and len(names) == 1, (fmt, M, N, K, names)
+    assert "gemm_kernel" in names[0] or "rows_mfma_kernel" in names[0], (fmt, M, N, K, names)
+    return "gemm_kernel" in names[0]
+
+
+for N in (1, 96, 512, 1024):
+    for M in (8, 9, 12, 13, 16):
+        for K in (512, 1088, 1984, 2048, 2560, 4032, 4096, 6144):
+            for fmt in FMT:
+                want = {"nv4": M > (8 if 2048 <= K < 4096 else 12),
+                        "w6": M > 12 and K < 2048, "w8": M > 12 and K < 2048, "w8_f16": M > 12 and K < 2048,
+                        "mx8": False, "bf16": False}[fmt]
+                assert gemm(fmt, M, N, K) == want, (fmt, M, N, K, want)
+for fmt in FMT:
+    assert gemm(fmt, 13, 1025, 2112) and gemm(fmt, 9, 2000, 1088) and gemm(fmt, 13, 512, 10304)
+    if not fmt.startswith("w8"):
+        assert gemm(fmt, 13, 1025, 2112, 2)
+""")
