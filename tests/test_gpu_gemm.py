@@ -4,9 +4,11 @@ the shapes of up to 16 rows that fall to it.
 fp32 outputs lie within the MFMA accumulation bound of the exact (float64)
 sum (oracle.ordered.mfma_bound; a K split over up to 10 waves adds as many
 additions as a K split over 10 slices) and bf16 outputs are the same sums
-rounded.  Sizes sit at the edges of its row tiles (16, 32, 48, 64, 128),
-column tiles (16 .. 128), 128-value K units (K = 64 .. 1088, not multiples of
-128) and waves (more waves than units), with odd N.
+rounded.  Every tile shape runs in every format (TILES; test_routes.py checks
+on the CPU that these sizes take them), off the edges of its row tile (16 ..
+128), column tile (16 .. 128) and 128-value K units, with odd N, with fewer
+units than waves and with enough for the ring to wrap; other sizes sit at
+exact tiles and at the smallest ones.
 """
 import numpy as np
 import pytest
@@ -23,6 +25,25 @@ pytestmark = pytest.mark.gpu
 
 FMTS = ["mx8", "w8", "w8_f16", "w6", "nv4", "bf16"]
 
+# tile shape (MT, NT, WN, WK, D): sizes M, N, K that the launcher takes it for
+# in every format on 256 CUs (the 16-bit tails of an odd scale plane are at
+# K % 128 == 64 and N odd)
+TILES = {
+    (1, 1, 1, 8, 1): [(17, 33, 192), (31, 33, 1984)],
+    (1, 1, 1, 10, 2): [(17, 33, 1088), (31, 33, 3136)],
+    (1, 2, 1, 8, 1): [(33, 2049, 320), (33, 2049, 1984)],
+    (2, 1, 1, 8, 1): [(81, 1345, 320), (145, 801, 960)],
+    (2, 1, 4, 2, 3): [(17, 2049, 192), (17, 8193, 704)],
+    (2, 2, 1, 8, 1): [(17, 4097, 576), (17, 4097, 1984)],
+    (3, 1, 2, 4, 2): [(17, 4097, 320), (33, 4097, 1344)],
+    (3, 1, 4, 2, 2): [(33, 8193, 192), (33, 8193, 704)],
+    (4, 1, 4, 2, 2): [(50, 8193, 192), (50, 8193, 704)],
+    (4, 1, 8, 1, 2): [(50, 16385, 192), (50, 16385, 704)],
+    (8, 1, 8, 1, 2): [(65, 16385, 192), (100, 16385, 704)],
+}
+UP_TO_16 = [(3, 7001, 1920), (5, 1280, 2560), (9, 512, 2560), (13, 96, 1088), (16, 2560, 6144), (16, 2560, 640),
+            (16, 5000, 1984)]
+
 
 @pytest.fixture(scope="module")
 def F():
@@ -38,6 +59,22 @@ def planes_of(fmt, rng, n, k):
     return planes, w_op, gs
 
 
+def took(fmt, planes, gs, xd, N):
+    """fp4x_linear_rows's own result, or None where it leaves the call to the
+    16-row launches (a scale plane of under 4 bytes)."""
+    import _fp4x as B
+    code = {"mx8": B.FMT_MX8, "w8": B.FMT_W8_F32, "w8_f16": B.FMT_W8_F16, "w6": B.FMT_W6, "nv4": B.FMT_NV4,
+            "bf16": B.FMT_BF16}[fmt]
+    M, K = xd.shape
+    w1, s = (planes[1], planes[2]) if fmt == "w6" else (None, None if fmt == "bf16" else planes[1])
+    y = torch.empty((M, N), dtype=torch.float32, device=xd.device)
+    rc = B.lib().fp4x_linear_rows(code, B.ptr(xd), xd.stride(0), B.ptr(planes[0]), B.ptr(w1), B.ptr(s), gs, B.ptr(y),
+                                  B.DT_F32, M, N, K, B.stream_of(xd))
+    small = s is not None and s.numel() * s.element_size() < 4
+    assert rc == (B.NOT_TAKEN if small else B.OK), rc
+    return None if small else to_f32(y)
+
+
 def check(F, fmt, planes, w_op, gs, x, xd):
     base = "w8" if fmt == "w8_f16" else fmt
     y = to_f32(run(F, base, xd, planes, 1, torch.float32))
@@ -45,7 +82,19 @@ def check(F, fmt, planes, w_op, gs, x, xd):
     bound = ordered.mfma_bound(x, w_op, 10) * abs(gs)
     assert np.all(np.abs(y - exact) <= bound), (np.abs(y - exact) / bound).max()
     assert np.array_equal(bf16_bits(run(F, base, xd, planes, 1)), fm.bf16_bits(y))
+    if x.shape[0] > 16:
+        own = took(fmt, planes, gs, xd, y.shape[1])
+        assert own is None or np.array_equal(own.view(np.uint32), y.view(np.uint32)), "the blocked GEMM did not run"
     return y
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("M,N,K", [size for sizes in TILES.values() for size in sizes])
+def test_gemm_every_tile_shape(gpu, F, fmt, M, N, K):
+    rng = np.random.default_rng(M + N + K)
+    planes, w_op, gs = planes_of(fmt, rng, N, K)
+    x, _ = act(rng, M, K)
+    check(F, fmt, planes, w_op, gs, x, bf16_dev(x))
 
 
 @pytest.mark.parametrize("fmt", FMTS)
@@ -65,11 +114,10 @@ def test_gemm_rows(gpu, F, fmt, M, N, K):
 
 
 @pytest.mark.parametrize("fmt", FMTS)
-@pytest.mark.parametrize("M,N,K", [(3, 7001, 1920), (5, 1280, 2560), (9, 512, 2560), (13, 96, 1088), (16, 2560, 6144),
-                                   (16, 2560, 640), (16, 5000, 1984)])
+@pytest.mark.parametrize("M,N,K", UP_TO_16)
 def test_gemm_up_to_16_rows(gpu, F, fmt, M, N, K, monkeypatch):
-    """The shapes of up to 16 rows that fall to it, against the exact sums;
-    FP4X_GEMM=0 (the MFMA core or the few-rows kernel) stays within the same
+    """Shapes of up to 16 rows that fall to it (two of them in some formats only:
+    test_routes.py), against the exact sums; FP4X_GEMM=0 (the MFMA core or the few-rows kernel) stays within the same
     bound."""
     rng = np.random.default_rng(M + N + K)
     planes, w_op, gs = planes_of(fmt, rng, N, K)
@@ -91,6 +139,16 @@ def test_gemm_one_unit_rows(gpu, F, fmt, M, N):
     check(F, fmt, planes, w_op, gs, x, bf16_dev(x))
 
 
+@pytest.mark.parametrize("M,N", [(20, 260), (20, 261), (50, 16385)])
+def test_gemm_fp16_output(gpu, F, M, N):
+    """fp16 outputs are the fp32 ones rounded."""
+    rng = np.random.default_rng(N)
+    planes, _, _ = planes_of("w8", rng, N, 320)
+    xd = bf16_dev(act(rng, M, 320)[0])
+    y = run(F, "w8", xd, planes, 1, torch.float32)
+    assert torch.equal(run(F, "w8", xd, planes, 1, torch.float16), y.half())
+
+
 def test_gemm_bf16_short_tail(gpu, F):
     """K a multiple of 16 only (bf16)."""
     rng = np.random.default_rng(5)
@@ -101,13 +159,14 @@ def test_gemm_bf16_short_tail(gpu, F):
     assert np.all(np.abs(y - ordered.exact_sum(x, w_op)) <= ordered.mfma_bound(x, w_op, 10))
 
 
-@pytest.mark.parametrize("M", [3, 20, 70])
-def test_gemm_special_values(gpu, F, M):
+@pytest.mark.parametrize("M,N,K", [(3, 3001, 1088), (20, 3001, 1088), (70, 3001, 1088), (33, 8193, 704),
+                                   (50, 16385, 704)])
+def test_gemm_special_values(gpu, F, M, N, K):
     """MXFP8 exponent 255 (scale +inf) gives +-inf or NaN in its own columns
     only, NaN and inf activations reach their own rows only, as one launch per
-    16 rows gives them; K not a multiple of 128, N odd."""
+    16 rows gives them; K not a multiple of 128, N odd; K parts in 8, 2 and no
+    other waves."""
     rng = np.random.default_rng(M)
-    N, K = 3001, 1088                                # few rows of 64 tiles, many units
     (w, s), _, _ = prep("mx8", rng, N, K)
     s = s.clone()
     s[7, 3] = 255

@@ -1,8 +1,11 @@
 """Which kernel a dense linear launches, without a GPU (tests/standin.py, 256
-CUs): the path switches, and the mixer's up projection."""
+CUs): the path switches, the mixer's up projection, the lines between the
+few-rows kernels and the blocked GEMM, and the tile shapes that the GEMM's GPU
+tests mean to run."""
 import pytest
 
 import standin
+from test_gpu_gemm import TILES, UP_TO_16
 
 
 @pytest.fixture(scope="module")
@@ -77,4 +80,30 @@ for fmt in FMT:
     assert gemm(fmt, 13, 1025, 2112) and gemm(fmt, 9, 2000, 1088) and gemm(fmt, 13, 512, 10304)
     if not fmt.startswith("w8"):
         assert gemm(fmt, 13, 1025, 2112, 2)
+""")
+
+
+def test_gpu_gemm_sizes_take_their_tiles(route):
+    """The sizes of test_gpu_gemm.py take the tile shapes and kernels that it
+    says, in every format."""
+    route(f"TILES, UP_TO_16 = {TILES!r}, {UP_TO_16!r}" + r"""
+import re
+
+
+def tile(names):
+    return tuple(int(v) for v in re.findall(r"Li(\d+)E", re.search(r"gemm_kernel\S*?((?:Li\d+E){5})", names[0]).group(1)))
+
+
+for want, sizes in TILES.items():
+    for M, N, K in sizes:
+        for fmt in FMT:
+            rc, names = rows(fmt, M, N, K)
+            assert rc == B.OK and tile(names) == want, (fmt, M, N, K, names, want)
+some = {(9, 512, 2560): ("nv4",), (13, 96, 1088): ("w8", "w8_f16", "w6", "nv4")}
+for size in UP_TO_16:
+    for fmt in FMT:
+        rc, names = linear(fmt, *size)
+        assert rc == B.OK and ("gemm_kernel" in names[0]) == (fmt in some.get(size, FMT)), (fmt, size, names)
+# exponent 255 of MXFP8 with K parts in 8, 2 and no other waves
+assert [tile(rows("mx8", *s)[1])[3] for s in ((20, 3001, 1088), (33, 8193, 704), (50, 16385, 704))] == [8, 2, 1]
 """)
