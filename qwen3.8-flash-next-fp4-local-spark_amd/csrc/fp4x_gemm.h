@@ -223,7 +223,8 @@ template <> struct GemmUnit<FmtMX8> {
           : "=&v"(r[0].q[0]), "=&v"(r[0].q[1]), "=&v"(r[0].e)
           : "v"(a0), "v"(a1), "v"(sa) : "memory");
     }
-    else if constexpr (NT == 2) {
+    else {
+      static_assert(NT == 2, "strips per wave");
       asm volatile(
           "ds_read_b128 %0, %6\n\t"
           "ds_read_b128 %1, %7\n\t"
@@ -234,25 +235,6 @@ template <> struct GemmUnit<FmtMX8> {
           "s_waitcnt lgkmcnt(0)"
           : "=&v"(r[0].q[0]), "=&v"(r[0].q[1]), "=&v"(r[0].e), "=&v"(r[1].q[0]), "=&v"(r[1].q[1]), "=&v"(r[1].e)
           : "v"(a0), "v"(a1), "v"(sa), "n"(1 * BYTES) : "memory");
-    }
-    else {
-      static_assert(NT == 4, "strips per wave");
-      asm volatile(
-          "ds_read_b128 %0, %12\n\t"
-          "ds_read_b128 %1, %13\n\t"
-          "ds_read_u8 %2, %14\n\t"
-          "ds_read_b128 %3, %12 offset:%15\n\t"
-          "ds_read_b128 %4, %13 offset:%15\n\t"
-          "ds_read_u8 %5, %14 offset:%15\n\t"
-          "ds_read_b128 %6, %12 offset:%16\n\t"
-          "ds_read_b128 %7, %13 offset:%16\n\t"
-          "ds_read_u8 %8, %14 offset:%16\n\t"
-          "ds_read_b128 %9, %12 offset:%17\n\t"
-          "ds_read_b128 %10, %13 offset:%17\n\t"
-          "ds_read_u8 %11, %14 offset:%17\n\t"
-          "s_waitcnt lgkmcnt(0)"
-          : "=&v"(r[0].q[0]), "=&v"(r[0].q[1]), "=&v"(r[0].e), "=&v"(r[1].q[0]), "=&v"(r[1].q[1]), "=&v"(r[1].e), "=&v"(r[2].q[0]), "=&v"(r[2].q[1]), "=&v"(r[2].e), "=&v"(r[3].q[0]), "=&v"(r[3].q[1]), "=&v"(r[3].e)
-          : "v"(a0), "v"(a1), "v"(sa), "n"(1 * BYTES), "n"(2 * BYTES), "n"(3 * BYTES) : "memory");
     }
   }
   __device__ static uint32_t scale_off(const PlaneArgs& a, int64_t n) { return (uint32_t)(n * (a.K / 32)); }
@@ -305,7 +287,8 @@ template <bool F16S> struct GemmUnit<FmtW8<F16S>> {
           : "=&v"(r[0].q[0]), "=&v"(r[0].q[1]), "=&v"(r[0].e)
           : "v"(a0), "v"(a1), "v"(sa) : "memory");
     }
-    else if constexpr (NT == 2) {
+    else {
+      static_assert(NT == 2, "strips per wave");
       asm volatile(
           "ds_read_b128 %0, %6\n\t"
           "ds_read_b128 %1, %7\n\t"
@@ -317,25 +300,6 @@ template <bool F16S> struct GemmUnit<FmtW8<F16S>> {
           : "=&v"(r[0].q[0]), "=&v"(r[0].q[1]), "=&v"(r[0].e), "=&v"(r[1].q[0]), "=&v"(r[1].q[1]), "=&v"(r[1].e)
           : "v"(a0), "v"(a1), "v"(sa), "n"(1 * BYTES) : "memory");
     }
-    else {
-      static_assert(NT == 4, "strips per wave");
-      asm volatile(
-          "ds_read_b128 %0, %12\n\t"
-          "ds_read_b128 %1, %13\n\t"
-          "ds_read_u16 %2, %14\n\t"
-          "ds_read_b128 %3, %12 offset:%15\n\t"
-          "ds_read_b128 %4, %13 offset:%15\n\t"
-          "ds_read_u16 %5, %14 offset:%15\n\t"
-          "ds_read_b128 %6, %12 offset:%16\n\t"
-          "ds_read_b128 %7, %13 offset:%16\n\t"
-          "ds_read_u16 %8, %14 offset:%16\n\t"
-          "ds_read_b128 %9, %12 offset:%17\n\t"
-          "ds_read_b128 %10, %13 offset:%17\n\t"
-          "ds_read_u16 %11, %14 offset:%17\n\t"
-          "s_waitcnt lgkmcnt(0)"
-          : "=&v"(r[0].q[0]), "=&v"(r[0].q[1]), "=&v"(r[0].e), "=&v"(r[1].q[0]), "=&v"(r[1].q[1]), "=&v"(r[1].e), "=&v"(r[2].q[0]), "=&v"(r[2].q[1]), "=&v"(r[2].e), "=&v"(r[3].q[0]), "=&v"(r[3].q[1]), "=&v"(r[3].e)
-          : "v"(a0), "v"(a1), "v"(sa), "n"(1 * BYTES), "n"(2 * BYTES), "n"(3 * BYTES) : "memory");
-    }
     } else {
     if constexpr (NT == 1) {
       asm volatile(
@@ -346,7 +310,8 @@ template <bool F16S> struct GemmUnit<FmtW8<F16S>> {
           : "=&v"(r[0].q[0]), "=&v"(r[0].q[1]), "=&v"(r[0].e)
           : "v"(a0), "v"(a1), "v"(sa) : "memory");
     }
-    else if constexpr (NT == 2) {
+    else {
+      static_assert(NT == 2, "strips per wave");
       asm volatile(
           "ds_read_b128 %0, %6\n\t"
           "ds_read_b128 %1, %7\n\t"
@@ -357,25 +322,6 @@ template <bool F16S> struct GemmUnit<FmtW8<F16S>> {
           "s_waitcnt lgkmcnt(0)"
           : "=&v"(r[0].q[0]), "=&v"(r[0].q[1]), "=&v"(r[0].e), "=&v"(r[1].q[0]), "=&v"(r[1].q[1]), "=&v"(r[1].e)
           : "v"(a0), "v"(a1), "v"(sa), "n"(1 * BYTES) : "memory");
-    }
-    else {
-      static_assert(NT == 4, "strips per wave");
-      asm volatile(
-          "ds_read_b128 %0, %12\n\t"
-          "ds_read_b128 %1, %13\n\t"
-          "ds_read_b32 %2, %14\n\t"
-          "ds_read_b128 %3, %12 offset:%15\n\t"
-          "ds_read_b128 %4, %13 offset:%15\n\t"
-          "ds_read_b32 %5, %14 offset:%15\n\t"
-          "ds_read_b128 %6, %12 offset:%16\n\t"
-          "ds_read_b128 %7, %13 offset:%16\n\t"
-          "ds_read_b32 %8, %14 offset:%16\n\t"
-          "ds_read_b128 %9, %12 offset:%17\n\t"
-          "ds_read_b128 %10, %13 offset:%17\n\t"
-          "ds_read_b32 %11, %14 offset:%17\n\t"
-          "s_waitcnt lgkmcnt(0)"
-          : "=&v"(r[0].q[0]), "=&v"(r[0].q[1]), "=&v"(r[0].e), "=&v"(r[1].q[0]), "=&v"(r[1].q[1]), "=&v"(r[1].e), "=&v"(r[2].q[0]), "=&v"(r[2].q[1]), "=&v"(r[2].e), "=&v"(r[3].q[0]), "=&v"(r[3].q[1]), "=&v"(r[3].e)
-          : "v"(a0), "v"(a1), "v"(sa), "n"(1 * BYTES), "n"(2 * BYTES), "n"(3 * BYTES) : "memory");
     }
     }
   }
@@ -432,7 +378,8 @@ template <> struct GemmUnit<FmtW6> {
           : "=&v"(r[0].lo), "=&v"(r[0].hi), "=&v"(r[0].e)
           : "v"(a0), "v"(a1), "v"(sa) : "memory");
     }
-    else if constexpr (NT == 2) {
+    else {
+      static_assert(NT == 2, "strips per wave");
       asm volatile(
           "ds_read_b128 %0, %6\n\t"
           "ds_read_b64 %1, %7\n\t"
@@ -443,25 +390,6 @@ template <> struct GemmUnit<FmtW6> {
           "s_waitcnt lgkmcnt(0)"
           : "=&v"(r[0].lo), "=&v"(r[0].hi), "=&v"(r[0].e), "=&v"(r[1].lo), "=&v"(r[1].hi), "=&v"(r[1].e)
           : "v"(a0), "v"(a1), "v"(sa), "n"(1 * BYTES) : "memory");
-    }
-    else {
-      static_assert(NT == 4, "strips per wave");
-      asm volatile(
-          "ds_read_b128 %0, %12\n\t"
-          "ds_read_b64 %1, %13\n\t"
-          "ds_read_u16 %2, %14\n\t"
-          "ds_read_b128 %3, %12 offset:%15\n\t"
-          "ds_read_b64 %4, %13 offset:%15\n\t"
-          "ds_read_u16 %5, %14 offset:%15\n\t"
-          "ds_read_b128 %6, %12 offset:%16\n\t"
-          "ds_read_b64 %7, %13 offset:%16\n\t"
-          "ds_read_u16 %8, %14 offset:%16\n\t"
-          "ds_read_b128 %9, %12 offset:%17\n\t"
-          "ds_read_b64 %10, %13 offset:%17\n\t"
-          "ds_read_u16 %11, %14 offset:%17\n\t"
-          "s_waitcnt lgkmcnt(0)"
-          : "=&v"(r[0].lo), "=&v"(r[0].hi), "=&v"(r[0].e), "=&v"(r[1].lo), "=&v"(r[1].hi), "=&v"(r[1].e), "=&v"(r[2].lo), "=&v"(r[2].hi), "=&v"(r[2].e), "=&v"(r[3].lo), "=&v"(r[3].hi), "=&v"(r[3].e)
-          : "v"(a0), "v"(a1), "v"(sa), "n"(1 * BYTES), "n"(2 * BYTES), "n"(3 * BYTES) : "memory");
     }
   }
   __device__ static uint32_t scale_off(const PlaneArgs& a, int64_t n) { return (uint32_t)(n * (a.K / 16)); }
@@ -506,7 +434,8 @@ template <> struct GemmUnit<FmtNV4> {
           : "=&v"(r[0].q), "=&v"(r[0].e)
           : "v"(a0), "v"(sa) : "memory");
     }
-    else if constexpr (NT == 2) {
+    else {
+      static_assert(NT == 2, "strips per wave");
       asm volatile(
           "ds_read_b128 %0, %4\n\t"
           "ds_read_u16 %1, %5\n\t"
@@ -515,21 +444,6 @@ template <> struct GemmUnit<FmtNV4> {
           "s_waitcnt lgkmcnt(0)"
           : "=&v"(r[0].q), "=&v"(r[0].e), "=&v"(r[1].q), "=&v"(r[1].e)
           : "v"(a0), "v"(sa), "n"(1 * BYTES) : "memory");
-    }
-    else {
-      static_assert(NT == 4, "strips per wave");
-      asm volatile(
-          "ds_read_b128 %0, %8\n\t"
-          "ds_read_u16 %1, %9\n\t"
-          "ds_read_b128 %2, %8 offset:%10\n\t"
-          "ds_read_u16 %3, %9 offset:%10\n\t"
-          "ds_read_b128 %4, %8 offset:%11\n\t"
-          "ds_read_u16 %5, %9 offset:%11\n\t"
-          "ds_read_b128 %6, %8 offset:%12\n\t"
-          "ds_read_u16 %7, %9 offset:%12\n\t"
-          "s_waitcnt lgkmcnt(0)"
-          : "=&v"(r[0].q), "=&v"(r[0].e), "=&v"(r[1].q), "=&v"(r[1].e), "=&v"(r[2].q), "=&v"(r[2].e), "=&v"(r[3].q), "=&v"(r[3].e)
-          : "v"(a0), "v"(sa), "n"(1 * BYTES), "n"(2 * BYTES), "n"(3 * BYTES) : "memory");
     }
   }
   __device__ static uint32_t scale_off(const PlaneArgs& a, int64_t n) { return (uint32_t)(n * (a.K / 16)); }
