@@ -217,6 +217,7 @@ int fp4x_mx8_linear(const void* x, int64_t x_stride, const void* w, const void* 
   p.pa.s = static_cast<const uint8_t*>(s);
   if (launch_rows_wide<FmtMX8>(p, (hipStream_t)stream)) return check_launch("mx8_rows");    // 16-20 rows per CU, M = 1
   if (launch_mx8_stream_entry(p, (hipStream_t)stream)) return check_launch("mx8_stream");   // many tiles
+  if (gemm_few_rows(p, FP4X_FMT_MX8) && launch_gemm_mx8(p, (hipStream_t)stream)) return check_launch("mx8_gemm");
   if (launch_rows_gemv<FmtMX8>(p, 1, (hipStream_t)stream)) return check_launch("mx8_rows");  // fewer rows
   if (launch_mx8_stream_tile_entry(p, (hipStream_t)stream)) return check_launch("mx8_stream"); // 1/2-1 tile per CU
   if ((ksplit == 1 || gemm_few_tiles(p)) && launch_gemm_mx8(p, (hipStream_t)stream)) return check_launch("mx8_gemm");
@@ -231,6 +232,7 @@ int fp4x_bf16_linear(const void* x, int64_t x_stride, const void* w, void* out, 
   if (M == 0 || N == 0) return FP4X_OK;
   GemvLaunch p = base_launch(FP4X_FMT_BF16, x, x_stride, out, out_dtype, N, M, N, K, ksplit, part, tickets);
   p.pa.w0 = static_cast<const uint8_t*>(w);
+  if (gemm_few_rows(p, FP4X_FMT_BF16) && launch_gemm_bf16(p, (hipStream_t)stream)) return check_launch("bf16_gemm");
   if (launch_rows_gemv<FmtBF16>(p, 1, (hipStream_t)stream)) return check_launch("bf16_rows");
   if ((ksplit == 1 || gemm_few_tiles(p)) && launch_gemm_bf16(p, (hipStream_t)stream)) return check_launch("bf16_gemm");
   return launch_gemv_mfma<FmtBF16, EpiStore>(p, 1, (hipStream_t)stream);

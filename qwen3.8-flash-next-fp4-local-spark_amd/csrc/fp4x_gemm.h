@@ -878,28 +878,28 @@ inline bool gemm_small(const GemvLaunch& p) {
   return tiles * 2 < device_cus() && p.M > (p.pa.K < 2048 ? 12 : 8) && (p.ksplit == 1 || p.pa.K <= 4096);
 }
 
-// Those of the few-rows kernels' shapes that this kernel takes first.  us with
-// weights from HBM (64 matrices, 1 GB written before each replay), few-rows
-// kernel / this, [512 x K]:
-//   K               M = 13, 1088   2560         4096         6144
-//   NVFP4           5.13 / 4.41    6.02 / 5.53  7.20 / 6.92  8.88 / 8.77
-//   W6              5.22 / 4.81    6.17 / 6.50  7.48 / 7.77  9.26 / 10.00
-//   MXFP8           4.85 / 4.85    5.95 / 5.95  7.19 / 7.67  8.99 / 9.74
-//   bf16            4.88 / 4.95    6.09 / 6.51  7.32 / 7.86  9.06 / 10.11
-// NVFP4 at M = 9: 2560 5.63 / 5.27, 4096 6.55 / 6.92, 6144 7.95 / 8.72; the
-// other formats lose up to a quarter there.  W8 stands between W6 and MXFP8
-// (M = 13: 0.93-1.02 of the few-rows time below K = 2048, 1.01-1.08 beyond).
-// N from 48 to 1016 moves none of these by more than a few percent.  MXFP8
-// and bf16 are at 0.95-1.05 at best (M = 16), so their few-rows kernel stays.
+// Those of the few-rows kernels' shapes that this kernel takes first: from M
+// on by format and K, since its time goes up in steps of its K parts and hardly
+// with M, and theirs with K and M.  us with weights from HBM (graph replays of
+// up to 64 matrices, 1 GB read before each), few-rows kernel / this, [512 x K]
+// at M = 9, 13 and 16:
+//   K       1088                             2560                             6144
+//   NVFP4   4.8 / 4.3  5.0 / 4.3  5.2 / 4.4  5.5 / 5.2  6.0 / 5.3  6.2 / 5.7  7.8 / 8.4  8.8 / 8.5  9.5 / 8.6
+//   W6      4.8 / 4.6  5.1 / 4.7  5.3 / 4.8  5.6 / 5.9  6.1 / 6.3  6.3 / 6.4  8.1 / 9.5  9.1 / 9.6  9.8 / 9.7
+//   W8      4.5 / 4.5  4.7 / 4.6  4.9 / 4.7  5.5 / 5.5  5.9 / 5.8  6.1 / 6.0  8.1 / 9.2  9.0 / 9.3  9.6 / 9.4
+//   MXFP8   4.5 / 4.6  4.7 / 4.7  4.9 / 4.8  5.5 / 5.4  5.8 / 5.7  6.1 / 6.0  7.9 / 9.2  8.9 / 9.3  9.5 / 9.5
+//   bf16    4.6 / 4.6  4.8 / 4.8  5.0 / 4.8  5.5 / 5.8  5.9 / 6.0  6.2 / 6.2  8.0 / 9.0  9.1 / 9.4  9.7 / 9.7
+// Over 16 K from 512 to 8192, N = 96, 512 and 1000 and M from 9 to 16 these
+// lines cost 0.8-1.4% against the better of the two on average and 10% at worst
+// (14% for NVFP4 below K = 2048 at 9 to 12 rows).
 inline bool gemm_before_rows(const GemvLaunch& p, int fmt) {
-  if (!gemm_small(p)) return false;
-  switch (fmt) {
-    case FP4X_FMT_NV4: return p.pa.K < 4096 || p.M > 12;
-    case FP4X_FMT_W6:
-    case FP4X_FMT_W8_F32:
-    case FP4X_FMT_W8_F16: return p.pa.K < 2048;
-    default: return false;
-  }
+  const int K = p.pa.K;
+  const int above = fmt == FP4X_FMT_NV4   ? K < 2048 ? 12 : K < 4096 ? 8 : 10
+                    : K >= 4096           ? 14
+                    : K >= 2048           ? 10
+                    : fmt == FP4X_FMT_MX8 ? 16
+                                          : 12;
+  return gemm_small(p) && p.M > above;
 }
 
 }  // namespace fp4x

@@ -69,13 +69,11 @@ def gemm(fmt, M, N, K, ks=1):
 
 
 for N in (1, 96, 512, 1024):
-    for M in (8, 9, 12, 13, 16):
+    for M in range(5, 17):
         for K in (512, 1088, 1984, 2048, 2560, 4032, 4096, 6144):
             for fmt in FMT:
-                want = {"nv4": M > (8 if 2048 <= K < 4096 else 12),
-                        "w6": M > 12 and K < 2048, "w8": M > 12 and K < 2048, "w8_f16": M > 12 and K < 2048,
-                        "mx8": False, "bf16": False}[fmt]
-                assert gemm(fmt, M, N, K) == want, (fmt, M, N, K, want)
+                above = {"nv4": (12, 8, 10), "mx8": (16, 10, 14)}.get(fmt, (12, 10, 14))[(K >= 2048) + (K >= 4096)]
+                assert gemm(fmt, M, N, K) == (M > above), (fmt, M, N, K, above)
 for fmt in FMT:
     assert gemm(fmt, 13, 1025, 2112) and gemm(fmt, 9, 2000, 1088) and gemm(fmt, 13, 512, 10304)
     if not fmt.startswith("w8"):
@@ -99,7 +97,7 @@ for want, sizes in TILES.items():
         for fmt in FMT:
             rc, names = rows(fmt, M, N, K)
             assert rc == B.OK and tile(names) == want, (fmt, M, N, K, names, want)
-some = {(9, 512, 2560): ("nv4",), (13, 96, 1088): ("w8", "w8_f16", "w6", "nv4")}
+some = {(9, 512, 2560): ("nv4",), (13, 96, 1088): ("w8", "w8_f16", "w6", "nv4", "bf16")}
 for size in UP_TO_16:
     for fmt in FMT:
         rc, names = linear(fmt, *size)
