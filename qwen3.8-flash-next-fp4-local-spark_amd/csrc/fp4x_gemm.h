@@ -6,7 +6,8 @@
 // It serves more than 16 rows, which the other kernels take as one launch per
 // 16 rows (each reading every weight again), and the shapes of up to 16 rows
 // that only the MFMA core took (rows too few or too long for the streaming
-// kernels, K not a multiple of 512).
+// kernels, K not a multiple of 512), and some of the few-rows kernels' shapes
+// at 9 to 16 rows (gemm_before_rows).
 //
 // A workgroup owns a tile of 16 MT rows of x and 16 NT WN rows of w.  Its WN x
 // WK waves split the tile's columns WN ways and K WK ways.  K advances in
@@ -27,16 +28,19 @@
 // or registers, took 37-41 and were slower on every narrower matrix; torch's
 // bf16 product of that size takes 41 with its weights from HBM.
 //
-// us per call, graph replays from HBM, one launch per 16 rows -> this:
+// us per call with weights from HBM (graph replays of 8 to 64 calls on weights
+// of their own, 1 GB read before each), one launch per 16 rows -> this:
 //   M                     24          64          256
-//   MXFP8 [16384 x 2560]  22 -> 13    42 -> 19    164 -> 38
-//   MXFP8 [2560 x 6144]   24 -> 11    65 -> 15    255 -> 28
-//   W6 [1280 x 2560]      19 -> 5.7   41 -> 6.6   164 -> 10
-//   NVFP4 [13312 x 2560]  17 -> 11    36 -> 16    143 -> 37
-//   W8 [2560 x 640]       11 -> 4.2   24 -> 4.7   92 -> 6.1
-// and against the core at M = 16: [5000 x 1920] 11-13 -> 5.9-6.8, [2560 x
-// 6144] 15-18 -> 8.7-9.9, [1280 x 2560] 8.4-10.9 -> 4.6-6.0, [2560 x 640]
-// 6.0-7.9 -> 3.5-3.7.
+//   MXFP8 [16384 x 2560]  23 -> 14    44 -> 21    169 -> 39
+//   MXFP8 [2560 x 6144]   25 -> 12    67 -> 16    263 -> 29
+//   W6 [1280 x 2560]      21 -> 6.1   51 -> 7.1   202 -> 11
+//   NVFP4 [13312 x 2560]  18 -> 12    38 -> 17    145 -> 39
+//   W8 [2560 x 640]       12 -> 4.8   26 -> 5.4   112 -> 6.9
+// and against the core: at M = 16 [5000 x 1920] 12-13 -> 6.8-8.3, [2560 x 6144]
+// 17-19 -> 10, [1280 x 2560] 9-12 -> 5.8-6.5, [2560 x 640] 6.7-9.0 -> 4.1-4.3;
+// at M = 1, 2 and 4 [9000 x 1088] 12-16 -> 7.0-9.1.  Over 29 to 107 such calls
+// per row count from 1 to 16 it takes 0.64 to 0.70 of the core's time, 0.92 at
+// most (K = 1088 to 4160, 2100 to 16000 rows).
 #pragma once
 #include <type_traits>
 #include "fp4x_stream.h"
@@ -805,14 +809,14 @@ bool launch_gemm_cfg(const GemvLaunch& p, hipStream_t st) {
   return true;
 }
 
-// Estimated us of a call with tile shape C, good enough to choose by: fitted
-// to 9,000 timings (5 formats x 10 matrices from [96 x 2560] to [16384 x 2560]
-// and [2560 x 6144] x 14 row counts from 5 to 256 x 20 tile shapes), where the
-// choice among the shapes below takes 1.03 times the fastest one's time on
-// (geometric) average and 1.27 times at worst.  The busiest CU's workgroups
-// run in rounds of as many as its LDS holds; a step costs the longer of a
-// memory round trip over the stages in flight and the stage's bytes, then the
-// MFMAs and the decoding.
+// Estimated us of a call with tile shape C, good enough to choose by: over 450
+// calls (MXFP8, W8, W6, NVFP4 and bf16, 9 matrices from [96 x 2560] to [16384 x
+// 2560], 10 row counts from 17 to 256, weights from HBM) the shape that it
+// chooses takes 1.01 times the fastest one's time on (geometric) average and
+// 1.12 times at worst.  The busiest CU's workgroups run in rounds of as many as
+// its LDS holds; a step costs the longer of a memory round trip over the stages
+// in flight and the stage's bytes, then the MFMAs and the decoding; the five
+// constants are a fit to timings of 20 tile shapes.
 template <class F, class C>
 float gemm_cost(const GemvLaunch& p, int cus) {
   using S = GemmShape<F, C::MT, C::NT, C::WN, C::WK, C::D>;

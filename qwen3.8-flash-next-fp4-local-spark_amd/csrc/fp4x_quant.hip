@@ -17,9 +17,9 @@
 // on; exact_quot gives the same quotient in 3 from the scale's reciprocal, and
 // the INT2 codes need comparisons only.  Groups with infinities, NaN or scales
 // at the ends of their range still divide.  us, before -> after, kernels alone
-// (MXFP8 rows): the 248,320 x 2560 head's INT2 copy 396 -> 186 (893 MB);
-// [16384 x 2560] to W8 33 -> 15, to W6 34 -> 18, to NVFP4 44 -> 20, its
-// global maximum 99 -> 11 (one atomic per workgroup that raises it, instead
+// (MXFP8 rows, traced): the 248,320 x 2560 head's INT2 copy 416 -> 160 (893
+// MB); [16384 x 2560] to W8 35 -> 18, to W6 35 -> 20, to NVFP4 44 -> 20, its
+// global maximum 100 -> 14 (one atomic per workgroup that raises it, instead
 // of one per wave, all on one word).
 #include <cmath>
 

@@ -3,7 +3,7 @@
 * dequant: the bf16 operand each kernel decodes is bit-exact with the
   oracle's dequantize-then-round (all formats, all fp8 codes).
 * GEMV: |y - y_oracle| <= 1e-2 + 2e-3 |y_oracle| against the fp32-accumulated
-  oracle, for M = 1..20 (M > 16 runs as 16-row launches), split-K and tails;
+  oracle, for M = 1..20 (M > 16 runs the blocked GEMM), split-K and tails;
   and, in fp32, within the MFMA accumulation bound of the exact (float64)
   sum (oracle.ordered.mfma_bound).
 """
