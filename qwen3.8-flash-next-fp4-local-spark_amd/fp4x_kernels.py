@@ -129,7 +129,7 @@ def _linear(fn, fmt, x2, n, k, ks, out_dtype, args, planes, gs=1.0):
         return out
     if m > MAX_M:
         if ks > 1:  # unused here, but refused where the 16-row entry refuses it (M = 0 launches nothing)
-            _L.check(fn(_ptr(x2), x2.stride(0), *args, _ptr(out), _dt(out_dtype), 0, n, k, ks, _ptr(out), _ptr(out), st),
+            _L.check(fn(_ptr(x2), x2.stride(0), *args, _ptr(out), _dt(out_dtype), 0, n, k, ks, _ptr(x2), _ptr(x2), st),
                      fn.__name__)
         rc = _L.lib().fp4x_linear_rows(fmt, _ptr(x2), x2.stride(0), *planes, gs, _ptr(out), _dt(out_dtype), m, n, k, st)
         if rc == _L.OK:

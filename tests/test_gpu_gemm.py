@@ -224,7 +224,7 @@ def test_gemm_refuses_bad_k_splits(gpu, F, fmt, K, bk, ks):
     planes, _, _ = planes_of(fmt, rng, 32, K)
     x = bf16_dev(act(rng, 20, K)[0])
 
-    def call(m, bk, ks):
+    def call(m, bk, ks, planes=planes):
         cfg = (32, bk, 4, ks) if fmt == "nv4" else (32, bk, ks, 4)
         fn = {"mx8": F.mx8_linear, "w8": F.w8_linear, "w6": F.w6_linear, "nv4": F.nv4_linear, "bf16": F.bf16_linear}[fmt]
         return fn(x[:m], *planes, cfg)
@@ -232,3 +232,6 @@ def test_gemm_refuses_bad_k_splits(gpu, F, fmt, K, bk, ks):
         with pytest.raises(ValueError):
             call(m, bk, ks)
     assert call(20, 32, 2).shape == (20, 32)
+    none = [t[:0] if torch.is_tensor(t) else t for t in planes]
+    for m in (16, 20):                               # no weight rows
+        assert call(m, 32, 2, none).shape == (m, 0)
